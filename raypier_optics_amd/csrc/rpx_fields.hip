@@ -671,15 +671,6 @@ struct ExpCheb {
     }
 };
 
-// 1/sqrt(a): the hardware estimate (2^-24) and one third-order step
-// y (1 + e/2 + 3 e^2 / 8), e = 1 - a y^2, for the normal, finite, positive a
-// of the field sum.
-__device__ __forceinline__ double rsq_third(double a) {
-    const double y = __builtin_amdgcn_rsq(a);
-    const double e = fma(-(a * y), y, 1.0);
-    return fma(y * e, fma(e, 0.375, 0.5), y);
-}
-
 struct FieldAcc {
     double r0 = 0, i0 = 0, r1 = 0, i1 = 0, r2 = 0, i2 = 0;
     // += (ur + i ui) V, V the record's last factor

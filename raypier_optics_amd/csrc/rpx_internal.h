@@ -128,7 +128,33 @@ enum : uint32_t {
     V_FLAT = F_PLANE | F_DISTORT | M_SIMPLE | M_FRESNEL | M_GRATING
 };
 
+// 1/sqrt(a): the hardware estimate (2^-24) and one third-order step
+// y (1 + e/2 + 3 e^2 / 8), e = 1 - a y^2, for normal, finite, positive a
+// (within an ulp of the rounded value).
+RPX_DEV double rsq_third(double a) {
+    const double y = __builtin_amdgcn_rsq(a);
+    const double e = fma(-(a * y), y, 1.0);
+    return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
 // ------------------------------------------------------------------- scene
+// A Zernike distortion as the kernels evaluate it: `n` groups from `first`,
+// of at most `terms` coefficients per polynomial.
+struct ZTable {
+    double inv_radius;
+    int32_t first, n, terms, pad;
+};
+
+// The coefficients of one |m| whose sag polynomials have one parity, summed:
+// polynomials in r^2.  R and the sag carry one more factor r when `odd`, R'
+// and R/r when not.  _C: coefficients with m >= 0, _S: with m < 0.
+enum : int { ZG_SAG_C, ZG_SAG_S, ZG_R_C, ZG_R_S, ZG_RP_C, ZG_RP_S, ZG_ROR_C, ZG_ROR_S, ZG_POLYS };
+#define ZG_TERMS (RPX_ZPOLY / 2)
+struct ZGroup {
+    int32_t m, odd;
+    double p[ZG_POLYS][ZG_TERMS];
+};
+
 // Device view of an uploaded scene (pointers into one device allocation).
 struct SceneView {
     const rpx_face_list_t *face_lists;
@@ -136,11 +162,10 @@ struct SceneView {
     const rpx_material_t *materials;
     const rpx_shape_op_t *shape_ops;
     const double *vertices;
-    const rpx_zernike_t *zernikes;
-    const rpx_zernike_coef_t *zcoefs;
-    const rpx_zernike_insn_t *zinsns;
+    const ZTable *ztables;
+    const ZGroup *zgroups;
     int32_t n_face_lists, n_faces, n_materials, n_shape_ops, n_vertices;
-    int32_t n_zernikes, n_zcoefs, n_zinsns;
+    int32_t n_zernikes;
     int32_t n_list_faces;   // faces that belong to face lists (chain order)
     int32_t max_children;
 };

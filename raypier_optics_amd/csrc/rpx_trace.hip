@@ -193,6 +193,44 @@ static size_t push_table(std::vector<char> &blob, const T *src, int n) {
     return off;
 }
 
+// Groups of one distortion (ZGroup), by |m| and parity, ascending in |m|.  A
+// radial polynomial of a Zernike term has the parity of m and its R' and R/r
+// the other one, so each |m| gives one group; terms of the other parity,
+// which the ABI does not exclude, go to a second group of the same |m|.
+static ZTable group_zernike(const rpx_zernike_t &z, const rpx_zernike_coef_t *coefs, std::vector<ZGroup> &out) {
+    static const int poly_of[4] = {RPX_ZP_SAG, RPX_ZP_R, RPX_ZP_RP, RPX_ZP_ROR};
+    std::map<std::pair<int, int>, ZGroup> groups;
+    int terms = 1;
+    for (int k = 0; k < z.n_coefs; ++k) {
+        const rpx_zernike_coef_t &c = coefs[z.coef_begin + k];
+        const int am = c.m >= 0 ? c.m : -c.m;
+        for (int q = 0; q < 4; ++q)
+            for (int i = 0; i < RPX_ZPOLY; ++i) {
+                const double a = c.poly[poly_of[q]][i];
+                if (a == 0.0) continue;
+                const int odd = q < 2 ? (i & 1) : !(i & 1);
+                auto it = groups.find({am, odd});
+                if (it == groups.end()) {
+                    ZGroup g;
+                    memset(&g, 0, sizeof(g));
+                    g.m = am;
+                    g.odd = odd;
+                    it = groups.emplace(std::make_pair(am, odd), g).first;
+                }
+                it->second.p[2 * q + (c.m < 0 ? 1 : 0)][i / 2] += c.nval * a;
+                terms = std::max(terms, i / 2 + 1);
+            }
+    }
+    ZTable t;
+    t.inv_radius = 1.0 / z.unit_radius;
+    t.first = (int32_t)out.size();
+    t.n = (int32_t)groups.size();
+    t.terms = terms;
+    t.pad = 0;
+    for (const auto &g : groups) out.push_back(g.second);
+    return t;
+}
+
 // The device tables of every scene on one device come from one heap: 2 MiB
 // chunks carved into blocks, so creating and destroying a scene makes no
 // hipMalloc / hipFree (hipFree waits for the whole device: a serving job's
@@ -243,9 +281,11 @@ extern "C" rpx_status_t rpx_scene_create(const rpx_scene_desc_t *d, rpx_scene_t 
     size_t o_m = push_table(blob, d->materials, d->n_materials);
     size_t o_s = push_table(blob, d->shape_ops, d->n_shape_ops);
     size_t o_v = push_table(blob, d->vertices, 2 * d->n_vertices);
-    size_t o_z = push_table(blob, d->zernikes, d->n_zernikes);
-    size_t o_zc = push_table(blob, d->zernike_coefs, d->n_zernike_coefs);
-    size_t o_zi = push_table(blob, d->zernike_insns, d->n_zernike_insns);
+    std::vector<ZTable> ztables;
+    std::vector<ZGroup> zgroups;
+    for (int i = 0; i < d->n_zernikes; ++i) ztables.push_back(group_zernike(d->zernikes[i], d->zernike_coefs, zgroups));
+    size_t o_z = push_table(blob, ztables.data(), (int)ztables.size());
+    size_t o_zg = push_table(blob, zgroups.data(), (int)zgroups.size());
     blob.resize(((blob.size() + 255) & ~size_t(255)) + 256);
     int device = 0;
     HIP_TRY(hipGetDevice(&device));
@@ -265,17 +305,14 @@ extern "C" rpx_status_t rpx_scene_create(const rpx_scene_desc_t *d, rpx_scene_t 
     v.materials = (const rpx_material_t *)(dev + o_m);
     v.shape_ops = (const rpx_shape_op_t *)(dev + o_s);
     v.vertices = (const double *)(dev + o_v);
-    v.zernikes = (const rpx_zernike_t *)(dev + o_z);
-    v.zcoefs = (const rpx_zernike_coef_t *)(dev + o_zc);
-    v.zinsns = (const rpx_zernike_insn_t *)(dev + o_zi);
+    v.ztables = (const ZTable *)(dev + o_z);
+    v.zgroups = (const ZGroup *)(dev + o_zg);
     v.n_face_lists = d->n_face_lists;
     v.n_faces = d->n_faces;
     v.n_materials = d->n_materials;
     v.n_shape_ops = d->n_shape_ops;
     v.n_vertices = d->n_vertices;
     v.n_zernikes = d->n_zernikes;
-    v.n_zcoefs = d->n_zernike_coefs;
-    v.n_zinsns = d->n_zernike_insns;
     int nlist = 0, maxc = 0, nglob = 0;
     for (int l = 0; l < d->n_face_lists; ++l) nlist += d->face_lists[l].n_faces;
     v.n_list_faces = nlist;
