@@ -213,92 +213,86 @@ RPX_DEV V3 zernike_grad(const SceneView &S, int zi, double x, double y) {
     return zernike_grad_t<ZG_TERMS>(S.ztables[zi], S.zgroups, x, y);
 }
 
-// ----------------------------------------------------------- conic / asphere
-// intersect_conic (cfaces.pyx:1695-1747)
-RPX_DEV double intersect_conic(V3 a, V3 d, double curvature, double conic_const) {
-    double beta = 1 + conic_const;
-    double R = -curvature;
-    double b2 = beta * beta;
-    double A = b2 * (d.z * d.z) + beta * (d.x * d.x) + beta * (d.y * d.y);
-    double B = -2 * R * beta * d.z + 2 * a.x * beta * d.x + 2 * a.y * beta * d.y + 2 * a.z * b2 * d.z;
-    double C = -2 * R * a.z * beta + (a.x * a.x) * beta + (a.y * a.y) * beta + (a.z * a.z) * b2;
-    double D = B * B - 4 * A * C;
-    if (D < 0) return -1;
-    D = sqrt(D);
-    if (R * beta * d.z <= 0) return (-B + D) / (2 * A);
-    return (-B - D) / (2 * A);
-}
-
-// x^2 .. x^nmax into pw[2..nmax].  x^2 is the rounded product (the
-// reference's x**2); higher powers come from a double-double product chain
-// rounded once, i.e. correctly rounded like the C library's pow for these
-// integer exponents, at a fraction of pow's cost.
-RPX_DEV void pow_chain(double x, double *pw, int nmax) {
-    double hi = x * x;
-    double lo = fma(x, x, -hi);
-    pw[2] = hi;
-    for (int k = 3; k <= nmax; ++k) {
-        double p = hi * x;
-        double e = fma(hi, x, -p);
-        lo = fma(lo, x, e);
-        double s = p + lo;
-        lo = lo - (s - p);
-        hi = s;
-        pw[k] = hi + lo;
-    }
-}
-
-struct Asph {
-    double R, beta, A4, A6, A8, A10, A12, A14, A16, R3;
-    V3 a, d;
+// -------------------------------------------------------------- segments
+// A ray segment in a face list's frame: from p1 along the unit vector u for
+// slen.  The reference parametrises a segment by the fraction h of p2 - p1 and
+// scales the root it accepts by |p2 - p1|, for every face (cfaces.pyx); here a
+// face's test gives the distance itself, so that the length, the reciprocals
+// and the unit vector are formed once per face list (once for all lists that
+// share the global frame) and a plane costs a multiplication.  Roots agree
+// with the reference's to a few ulp of the segment.
+struct Seg {
+    V3 p1, u;
+    double slen, inv_uz;
 };
 
-// eval_aspheric_impf (cfaces.pyx:1854-1863)
-RPX_DEV double asph_impf(const Asph &A, double alpha) {
-    double tx = A.a.x + alpha * A.d.x, ty = A.a.y + alpha * A.d.y;
-    double r2 = (tx * tx + ty * ty);
-    double pw[9];
-    pow_chain(r2, pw, 8);
-    double out = r2;
-    out /= A.R * (1 + sqrt(1 - A.beta * r2 / (A.R * A.R)));
-    out -= A.a.z + alpha * A.d.z;
-    out += A.A4 * pw[2] + A.A6 * pw[3] + A.A8 * pw[4] + A.A10 * pw[5] + A.A12 * pw[6] + A.A14 * pw[7] +
-           A.A16 * pw[8];
-    return out;
+RPX_DEV Seg make_seg(V3 p1, V3 p2) {
+    Seg g;
+    const V3 s = sub(p2, p1);
+    g.p1 = p1;
+    g.slen = sqrt(fma(s.x, s.x, fma(s.y, s.y, s.z * s.z)));
+    g.u = mul(s, 1.0 / g.slen);
+    g.inv_uz = 1.0 / g.u.z;
+    return g;
 }
 
-// eval_aspheric_grad (cfaces.pyx:1866-1882)
-RPX_DEV double asph_grad(const Asph &A, double alpha) {
-    double tx = A.a.x + alpha * A.d.x, ty = A.a.y + alpha * A.d.y;
-    double r2 = (tx * tx + ty * ty);
-    double dx = A.d.x * tx;
-    double dy = A.d.y * ty;
-    double pw[8];
-    pow_chain(r2, pw, 7);
-    double out = A.A10 * (10 * dx + 10 * dy) * pw[4];
-    out += A.A12 * (12 * dx + 12 * dy) * pw[5];
-    out += A.A14 * (14 * dx + 14 * dy) * pw[6];
-    out += A.A16 * (16 * dx + 16 * dy) * pw[7];
-    out += A.A4 * (4 * dx + 4 * dy) * (r2);
-    out += A.A6 * (6 * dx + 6 * dy) * pw[2];
-    out += A.A8 * (8 * dx + 8 * dy) * pw[3] - A.d.z;
-    out += (2 * dx + 2 * dy) / (A.R * (sqrt(1 - A.beta * (r2) / (A.R * A.R)) + 1));
-    double s = sqrt(1 - A.beta * r2 / (A.R * A.R));
-    double s1 = s + 1;
-    out += A.beta * (2 * dx + 2 * dy) * (r2) / (2 * A.R3 * s * (s1 * s1));
-    return out;
+RPX_DEV V3 seg_at(const Seg &g, double t) {
+    return v3(fma(g.u.x, t, g.p1.x), fma(g.u.y, t, g.p1.y), fma(g.u.z, t, g.p1.z));
+}
+
+// Face list flags, set at scene creation in rpx_face_list_t.pad[0].
+enum : int { FL_INV_IDENTITY = 1, FL_TRANS_IDENTITY = 2 };
+
+RPX_DEV V3 to_local(const rpx_face_list_t &fl, V3 p) {
+    if (fl.pad[0] & FL_INV_IDENTITY) return p;
+    return transform(fl.inv_trans, p);
+}
+RPX_DEV V3 to_global_dir(const rpx_face_list_t &fl, V3 d) {
+    if (fl.pad[0] & FL_TRANS_IDENTITY) return d;
+    return rotate(fl.trans, d);
+}
+
+// ----------------------------------------------------------- conic / asphere
+// intersect_conic (cfaces.pyx:1695-1747) for a unit direction d: the distance.
+RPX_DEV double intersect_conic(V3 a, V3 d, double curvature, double conic_const) {
+    const double beta = 1 + conic_const;
+    const double R = -curvature;
+    const double b2 = beta * beta;
+    const double dt = fma(d.x, d.x, d.y * d.y), at = fma(a.x, a.x, a.y * a.y), ad = fma(a.x, d.x, a.y * d.y);
+    const double A = fma(b2, d.z * d.z, beta * dt);
+    // half of the reference's B
+    const double B = fma(beta, fma(-R, d.z, ad), b2 * (a.z * d.z));
+    const double C = fma(beta, fma(-2 * R, a.z, at), b2 * (a.z * a.z));
+    double D = fma(B, B, -(A * C));
+    if (D < 0) return -1;
+    D = sqrt(D);
+    return (R * beta * d.z <= 0 ? -B + D : -B - D) / A;
+}
+
+// x = r^2 polynomial A4 x^2 + .. + A16 x^8 and its derivative, by Horner's rule
+// (p[3..9] of an aspheric face).
+RPX_DEV double asph_poly(const rpx_face_t &f, double x) {
+    double v = f.p[9];
+#pragma unroll
+    for (int i = 8; i >= 3; --i) v = fma(v, x, f.p[i]);
+    return v * (x * x);
+}
+RPX_DEV double asph_dpoly(const rpx_face_t &f, double x) {
+    double v = 8 * f.p[9];
+#pragma unroll
+    for (int i = 8; i >= 3; --i) v = fma(v, x, (i - 1) * f.p[i]);
+    return v * x;
 }
 
 // A base-ray hit on an aspheric face is accepted only inside the aperture,
 // where the surface lies within z_height +/- p[12]; the converged root
 // satisfies the sag equation to within the Newton tolerance.  A segment whose
 // z-range misses that band cannot be accepted.
-RPX_DEV bool asph_outside_band(const rpx_face_t &f, V3 p1, V3 p2, int is_base) {
+RPX_DEV bool asph_outside_band(const rpx_face_t &f, const Seg &g, int is_base) {
     if (!is_base || f.p[12] < 0.0) return false;
-    double len = sep(p1, p2);
-    double m = f.p[12] + 1e-9 * (1.0 + fabs(f.p[1]) + f.p[12]) + 10.0 * f.p[10] * len * (1.0 + f.p[13]);
-    double zlo = fmin(p1.z, p2.z), zhi = fmax(p1.z, p2.z);
-    return zhi < f.p[1] - m || zlo > f.p[1] + m;
+    const double m = f.p[12] + 1e-9 * (1.0 + fabs(f.p[1]) + f.p[12]) + 10.0 * f.p[10] * g.slen * (1.0 + f.p[13]);
+    const double z2 = fma(g.u.z, g.slen, g.p1.z);
+    return fmax(g.p1.z, z2) < f.p[1] - m || fmin(g.p1.z, z2) > f.p[1] + m;
 }
 
 // A base ray's nearest-face search only accepts a face's hit closer than
@@ -334,56 +328,49 @@ RPX_DEV rpx_face_t face_uniform(const rpx_face_t *faces, int k) {
     return f;
 }
 
-// Base-face intersection used by DistortionFace (no recursion into a second
-// distortion level: the host refuses nested distortions).
+// Whether a root at distance t passes the reference's range test on h = t /
+// slen (tol <= h <= 1); false for NaN.
+RPX_DEV bool in_segment(const Seg &g, double t, double tol) { return t >= tol * g.slen && t <= g.slen; }
+
+// Base-face intersection, also used by DistortionFace (no recursion into a
+// second distortion level: the host refuses nested distortions).  Returns the
+// distance, or -1.
 template <uint32_t F>
-RPX_DEV double plain_intersect(const SceneView &S, const rpx_face_t &f, V3 p1, V3 p2, int is_base) {
+RPX_DEV double plain_intersect(const SceneView &S, const rpx_face_t &f, const Seg &g, int is_base) {
     const double tol = f.tolerance;
     switch (f.type) {
     case RPX_FACE_CIRCULAR: {
         if constexpr ((F & F_PLANE) == 0) return -1;  // cfaces.pyx:151-178
-        double max_length = sep(p1, p2);
-        double h = (f.p[2] - p1.z) / (p2.z - p1.z);
-        double d = f.p[0];
-        if ((h < tol) || (h > 1.0)) return -1;
-        double X = p1.x + h * (p2.x - p1.x) - f.p[1];
-        double Y = p1.y + h * (p2.y - p1.y);
-        if (is_base && (X * X + Y * Y) > (d * d / 4)) return -1;
-        return h * max_length;
+        const double t = (f.p[2] - g.p1.z) * g.inv_uz, d = f.p[0];
+        if (!in_segment(g, t, tol)) return -1;
+        const double X = fma(g.u.x, t, g.p1.x) - f.p[1], Y = fma(g.u.y, t, g.p1.y);
+        if (is_base && fma(X, X, Y * Y) > (d * d / 4)) return -1;
+        return t;
     }
     case RPX_FACE_SHAPED_PLANAR: {
         if constexpr ((F & F_PLANE) == 0) return -1;  // cfaces.pyx:201-226
-        double max_length = sep(p1, p2);
-        double h = (f.p[0] - p1.z) / (p2.z - p1.z);
-        if ((h < tol) || (h > 1.0)) return -1;
-        double X = p1.x + h * (p2.x - p1.x);
-        double Y = p1.y + h * (p2.y - p1.y);
-        if (is_base && !shape_inside(S, f.shape, X, Y)) return -1;
-        return h * max_length;
+        const double t = (f.p[0] - g.p1.z) * g.inv_uz;
+        if (!in_segment(g, t, tol)) return -1;
+        if (is_base && !shape_inside(S, f.shape, fma(g.u.x, t, g.p1.x), fma(g.u.y, t, g.p1.y))) return -1;
+        return t;
     }
     case RPX_FACE_RECTANGULAR: {
         if constexpr ((F & F_PLANE) == 0) return -1;  // cfaces.pyx:365-397
-        double max_length = sep(p1, p2);
-        double h = (f.p[3] - p1.z) / (p2.z - p1.z);
-        double lngth = f.p[0], wdth = f.p[1];
-        if ((h < tol) || (h > 1.0)) return -1;
+        const double t = (f.p[3] - g.p1.z) * g.inv_uz;
+        if (!in_segment(g, t, tol)) return -1;
         if (is_base) {
-            double X = p1.x + h * (p2.x - p1.x) - f.p[2];
-            double Y = p1.y + h * (p2.y - p1.y);
-            if (X * X > lngth * lngth / 4) return -1;
-            if (Y * Y > wdth * wdth / 4) return -1;
+            const double X = fma(g.u.x, t, g.p1.x) - f.p[2], Y = fma(g.u.y, t, g.p1.y);
+            if (X * X > f.p[0] * f.p[0] / 4) return -1;
+            if (Y * Y > f.p[1] * f.p[1] / 4) return -1;
         }
-        return h * max_length;
+        return t;
     }
     case RPX_FACE_POLYGON: {
         if constexpr ((F & F_PLANE) == 0) return -1;  // cfaces.pyx:1093-1108
-        double max_length = sep(p1, p2);
-        double h = (f.p[0] - p1.z) / (p2.z - p1.z);
-        if ((h < tol) || (h > 1.0)) return -1;
-        double X = p1.x + h * (p2.x - p1.x);
-        double Y = p1.y + h * (p2.y - p1.y);
-        if (is_base && polygon_face_inside(S.vertices + 2 * f.aux0, f.aux1, X, Y)) return h * max_length;
-        return -1;
+        const double t = (f.p[0] - g.p1.z) * g.inv_uz;
+        if (!is_base || !in_segment(g, t, tol)) return -1;
+        return polygon_face_inside(S.vertices + 2 * f.aux0, f.aux1, fma(g.u.x, t, g.p1.x), fma(g.u.y, t, g.p1.y))
+                   ? t : -1;
     }
     case RPX_FACE_SPHERICAL:
     case RPX_FACE_SHAPED_SPHERICAL: {
@@ -391,20 +378,17 @@ RPX_DEV double plain_intersect(const SceneView &S, const rpx_face_t &f, V3 p1, V
         const bool shaped = f.type == RPX_FACE_SHAPED_SPHERICAL;
         const double curvature = shaped ? f.p[0] : f.p[1];
         const double z_height = shaped ? f.p[1] : f.p[2];
-        V3 s = sub(p2, p1);
-        double cz = z_height - curvature;
-        V3 d = p1;
+        const double cz = z_height - curvature;
+        V3 d = g.p1;
         d.z -= cz;
-        double A = mag_sq(s);
-        double B = 2 * dot(s, d);
-        double C = mag_sq(d) - curvature * curvature;
-        double D = B * B - 4 * A * C;
+        // half of the reference's B, over |s|
+        const double B = fma(g.u.x, d.x, fma(g.u.y, d.y, g.u.z * d.z));
+        const double C = fma(d.x, d.x, fma(d.y, d.y, d.z * d.z)) - curvature * curvature;
+        double D = fma(B, B, -C);
         if (D < 0) return -1;
         D = sqrt(D);
-        double a1 = (-B + D) / (2 * A);
-        V3 pt1 = add(p1, mul(s, a1));
-        double a2 = (-B - D) / (2 * A);
-        V3 pt2 = add(p1, mul(s, a2));
+        double a1 = D - B, a2 = -B - D;
+        const V3 pt1 = seg_at(g, a1), pt2 = seg_at(g, a2);
         if (curvature >= 0) {
             if (pt1.z < cz) a1 = RPX_INF;
             if (pt2.z < cz) a2 = RPX_INF;
@@ -417,79 +401,77 @@ RPX_DEV double plain_intersect(const SceneView &S, const rpx_face_t &f, V3 p1, V
                 if (!shape_inside(S, f.shape, pt1.x, pt1.y)) a1 = RPX_INF;
                 if (!shape_inside(S, f.shape, pt2.x, pt2.y)) a2 = RPX_INF;
             } else {
-                double DD = f.p[0] * f.p[0] / 4.;
-                if ((pt1.x * pt1.x + pt1.y * pt1.y) > DD) a1 = RPX_INF;
-                if ((pt2.x * pt2.x + pt2.y * pt2.y) > DD) a2 = RPX_INF;
+                const double DD = f.p[0] * f.p[0] / 4.;
+                if (fma(pt1.x, pt1.x, pt1.y * pt1.y) > DD) a1 = RPX_INF;
+                if (fma(pt2.x, pt2.x, pt2.y * pt2.y) > DD) a2 = RPX_INF;
             }
         }
         if (a2 < a1) a1 = a2;
-        if (a1 > 1.0 || a1 < tol) return -1;
-        return a1 * sep(p1, p2);
+        return in_segment(g, a1, tol) ? a1 : -1;
     }
     case RPX_FACE_EXTRUDED_PLANAR: {
         if constexpr ((F & F_PLANE) == 0) return -1;  // cfaces.pyx:665-699
-        double ux = f.p[0], uy = f.p[1];
-        double vx = f.p[2] - ux, vy = f.p[3] - uy;
-        V3 s = sub(p2, p1);
-        double a;
+        const double ux = f.p[0], uy = f.p[1];
+        const double vx = f.p[2] - ux, vy = f.p[3] - uy;
+        const double den = fma(g.u.x, vy, -(g.u.y * vx));
+        const double ax = g.p1.x - ux, ay = g.p1.y - uy;
         if (is_base) {
-            a = (s.y * (ux - p1.x) - s.x * (uy - p1.y)) / (s.x * vy - s.y * vx);
-            if (a < 0) return -1;
-            if (a > 1) return -1;
+            // the position along the edge, num / den, must lie in 0..1
+            const double num = fma(g.u.x, ay, -(g.u.y * ax));
+            const double q = den < 0 ? -num : num;
+            if (q < 0 || q > fabs(den)) return -1;
         }
-        a = (vx * (p1.y - uy) - vy * (p1.x - ux)) / (s.x * vy - s.y * vx);
+        const double num = fma(vx, ay, -(vy * ax));
+        // behind the start: no division, where the caller would reject it
+        if (is_base && tol >= 0 && (den < 0 ? num > 0 : num < 0)) return -1;
+        const double t = num / den;
         if (is_base) {
-            double dz = a * (p2.z - p1.z);
-            double zz = p1.z + dz;
-            if (f.p[4] < zz && zz < f.p[5]) return a * mag(s);
-            return -1;
+            const double zz = fma(g.u.z, t, g.p1.z);
+            return f.p[4] < zz && zz < f.p[5] ? t : -1;
         }
-        return a * mag(s);
+        return t;
     }
     case RPX_FACE_CONIC: {
         if constexpr ((F & F_CONIC) == 0) return -1;  // cfaces.pyx:1767-1798
-        V3 d = sub(p2, p1);
-        V3 a = p1;
+        V3 a = g.p1;
         a.z -= f.p[1];
-        double a1 = intersect_conic(a, d, f.p[0], f.p[2]);
-        V3 pt1 = add(a, mul(d, a1));
-        if (is_base && !shape_inside(S, f.shape, pt1.x, pt1.y)) return -1;
-        if (a1 > 1.0 || a1 < tol) return -1;
-        return a1 * sep(p1, p2);
+        const double t = intersect_conic(a, g.u, f.p[0], f.p[2]);
+        if (is_base && !shape_inside(S, f.shape, fma(g.u.x, t, a.x), fma(g.u.y, t, a.y))) return -1;
+        return in_segment(g, t, tol) ? t : -1;
     }
     case RPX_FACE_ASPHERIC: {
         if constexpr ((F & F_ASPHERE) == 0) return -1;  // cfaces.pyx:1909-1976
-        double atol = f.p[10];
-        double tl = atol * atol;
-        if (asph_outside_band(f, p1, p2, is_base)) return -1;
-        V3 d = sub(p2, p1);
-        V3 a = p1;
+        if (asph_outside_band(f, g, is_base)) return -1;
+        // Newton from the conic's root on f(t) = r^2 / (R (1 + w)) + P(r^2) -
+        // (a.z + t u.z), w = sqrt(1 - beta r^2 / R^2); the conic term's
+        // derivative in r^2 is 1 / (2 R w) (the reference's two fractions,
+        // cfaces.pyx:1866-1882, added up), so a step takes one square root and
+        // one division.
+        const double atol = f.p[10] * g.slen;
+        const double tl = atol * atol;
+        V3 a = g.p1;
         a.z -= f.p[1];
-        double a1 = intersect_conic(a, d, f.p[0], f.p[2]);
-        Asph A;
-        A.R = -f.p[0];
-        A.beta = 1 + f.p[2];
-        A.A4 = f.p[3]; A.A6 = f.p[4]; A.A8 = f.p[5]; A.A10 = f.p[6];
-        A.A12 = f.p[7]; A.A14 = f.p[8]; A.A16 = f.p[9];
-        A.R3 = f.p[11];
-        A.a = a;
-        A.d = d;
-        double fv = asph_impf(A, a1), f_last = fv;
-        double dz = -fv / asph_grad(A, a1);
+        const double R = -f.p[0], k2 = (1 + f.p[2]) / (R * R);
+        double t = intersect_conic(a, g.u, f.p[0], f.p[2]);
+        double f_last = RPX_INF, dt = RPX_INF;
         bool converged = false;
-        for (int i = 0; i < 100; ++i) {
-            a1 += dz;
-            if (dz * dz < tl) { converged = true; break; }
-            fv = asph_impf(A, a1);
-            if (fabs(fv) > fabs(f_last)) return -1;
+        for (int i = 0; i <= 100; ++i) {
+            const double tx = fma(t, g.u.x, a.x), ty = fma(t, g.u.y, a.y);
+            const double r2 = fma(tx, tx, ty * ty);
+            const double w = sqrt(fma(-k2, r2, 1.0)), w1 = 1 + w;
+            const double inv = 1.0 / (R * w * w1);
+            const double fv = fma(r2 * w, inv, asph_poly(f, r2)) - fma(t, g.u.z, a.z);
+            if (i > 0 && fabs(fv) > fabs(f_last)) return -1;
             f_last = fv;
-            dz = -fv / asph_grad(A, a1);
+            const double slope = fma(w1, inv, 2 * asph_dpoly(f, r2));
+            dt = -fv / fma(fma(g.u.x, tx, g.u.y * ty), slope, -g.u.z);
+            if (i == 100) break;
+            t += dt;
+            if (dt * dt < tl) { converged = true; break; }
         }
         if (!converged) return -1;
-        V3 pt1 = add(a, mul(d, a1));
-        if (is_base && !shape_inside(S, f.shape, pt1.x, pt1.y)) return -1;
-        if (a1 > 1.0 || a1 < tol) return -1;
-        return a1 * sep(p1, p2);
+        if (is_base && !shape_inside(S, f.shape, fma(g.u.x, t, a.x), fma(g.u.y, t, a.y))) return -1;
+        return in_segment(g, t, tol) ? t : -1;
     }
     default:
         return -1;
@@ -519,7 +501,7 @@ RPX_DEV V3 plain_normal(const SceneView &S, const rpx_face_t &f, V3 p) {
             p.y = -p.y;
             p.x = -p.x;
         }
-        return norm(p);
+        return unit(p);
     }
     case RPX_FACE_EXTRUDED_PLANAR:  // cfaces.pyx:701-702
         return v3(f.p[6], f.p[7], f.p[8]);
@@ -537,32 +519,16 @@ RPX_DEV V3 plain_normal(const SceneView &S, const rpx_face_t &f, V3 p) {
         g.z *= sign;
         g.y *= sign;
         g.x *= sign;
-        return norm(g);
+        return unit(g);
     }
     case RPX_FACE_ASPHERIC: {
         if constexpr ((F & F_ASPHERE) == 0) return p;  // cfaces.pyx:1978-2007
-        double R = -f.p[0];
-        double beta = 1 + f.p[2];
-        int sign = f.invert_normals ? -1 : 1;
-        p.z -= f.p[1];
-        double r2 = p.x * p.x + p.y * p.y;
-        double root = sqrt(1 - (beta * (r2) / (R * R)));
-        double A4 = f.p[3], A6 = f.p[4], A8 = f.p[5], A10 = f.p[6], A12 = f.p[7], A14 = f.p[8], A16 = f.p[9];
-        double pw[8];
-        pow_chain(r2, pw, 7);
-        double df = 10 * A10 * pw[4] + 8 * A8 * pw[3] + 6 * A6 * pw[2] + 4 * A4 * r2;
-        df += 16 * A16 * pw[7] + 14 * A14 * pw[6] + 12 * A12 * pw[5];
-        df += 2 / (R * (1 + root));
-        double r1 = 1 + root;
-        df += beta * (r2) / (f.p[11] * root * (r1 * r1));
-        V3 g;
-        g.z = 1.0;
-        g.x = -df * p.x;
-        g.y = -df * p.y;
-        g.z *= sign;
-        g.y *= sign;
-        g.x *= sign;
-        return norm(g);
+        const double R = -f.p[0];
+        const int sign = f.invert_normals ? -1 : 1;
+        const double r2 = fma(p.x, p.x, p.y * p.y);
+        const double w = sqrt(fma(-(1 + f.p[2]) / (R * R), r2, 1.0));
+        const double df = 1.0 / (R * w) + 2 * asph_dpoly(f, r2);
+        return unit(v3(-df * p.x * sign, -df * p.y * sign, sign));
     }
     default:
         return p;
@@ -571,55 +537,49 @@ RPX_DEV V3 plain_normal(const SceneView &S, const rpx_face_t &f, V3 p) {
 
 // DistortionFace.intersect_c (cfaces.pyx:2339-2416)
 template <uint32_t F>
-RPX_DEV double distortion_intersect(const SceneView &S, const rpx_face_t &f, V3 p1, V3 p2) {
+RPX_DEV double distortion_intersect(const SceneView &S, const rpx_face_t &f, const Seg &g) {
     const rpx_face_t &face = S.faces[f.aux0];
     const int zi = f.aux1;
-    double a1, a2, h = sep(p2, p1);
-    double tolerance = f.p[0];
-    a2 = plain_intersect<F>(S, face, p1, p2, 0);
-    if (a2 > h || a2 < f.tolerance) return -1;
-    V3 d = sub(p2, p1);
-    V3 pt1 = add(p1, mul(d, a2 / h));
-    V3 dxdyz = zernike_grad(S, zi, pt1.x, pt1.y);
-    V3 n = plain_normal<F>(S, face, pt1);
-    pt1.z += dxdyz.z;
-    n.x /= n.z;
-    n.y /= n.z;
-    n.x -= dxdyz.x;
-    n.y -= dxdyz.y;
-    V3 o = sub(p1, pt1);
-    a1 = -h * dot(o, n) / dot(d, n);
-    if (a1 < fabs(dxdyz.z)) return -1;
+    double a1, a2;
+    const double tolerance = f.p[0];
+    a2 = plain_intersect<F>(S, face, g, 0);
+    if (a2 > g.slen || a2 < f.tolerance) return -1;
+    V3 pt1 = seg_at(g, a2);
+    // distance to the tangent plane of base + distortion at pt1
+    auto tangent_plane = [&](V3 &pt, double &dz) {
+        const V3 grad = zernike_grad(S, zi, pt.x, pt.y);
+        V3 n = plain_normal<F>(S, face, pt);
+        const double inv = 1.0 / n.z;
+        pt.z += grad.z;
+        dz = grad.z;
+        n.x = fma(n.x, inv, -grad.x);
+        n.y = fma(n.y, inv, -grad.y);
+        return -dot(sub(g.p1, pt), n) / dot(g.u, n);
+    };
+    double dz;
+    a1 = tangent_plane(pt1, dz);
+    if (a1 < fabs(dz)) return -1;
     for (int i = 0; i < 20; ++i) {
-        pt1 = add(p1, mul(d, a1 / h));
+        pt1 = seg_at(g, a1);
         if (fabs(a1 - a2) < tolerance) break;
-        double z_shift = zernike_sag(S, zi, pt1.x, pt1.y);
-        V3 q1 = p1, q2 = p2;
-        q1.z -= z_shift;
-        q2.z -= z_shift;
-        a2 = plain_intersect<F>(S, face, q1, q2, 0);
-        pt1 = add(q1, mul(d, a2 / h));
-        n = plain_normal<F>(S, face, pt1);
-        dxdyz = zernike_grad(S, zi, pt1.x, pt1.y);
-        pt1.z += dxdyz.z;
-        n.x /= n.z;
-        n.y /= n.z;
-        n.x -= dxdyz.x;
-        n.y -= dxdyz.y;
-        o = sub(p1, pt1);
+        Seg q = g;
+        q.p1.z -= zernike_sag(S, zi, pt1.x, pt1.y);
+        a2 = plain_intersect<F>(S, face, q, 0);
+        pt1 = seg_at(q, a2);
+        const double t = tangent_plane(pt1, dz);
         a2 = a1;
-        a1 = -h * dot(o, n) / dot(d, n);
+        a1 = t;
     }
     if (!shape_inside(S, f.shape, pt1.x, pt1.y)) return -1;
     return a1;
 }
 
 template <uint32_t F>
-RPX_DEV double face_intersect(const SceneView &S, const rpx_face_t &f, V3 p1, V3 p2, int is_base) {
+RPX_DEV double face_intersect(const SceneView &S, const rpx_face_t &f, const Seg &g, int is_base) {
     if constexpr ((F & F_DISTORT) != 0) {
-        if (f.type == RPX_FACE_DISTORTION) return distortion_intersect<F>(S, f, p1, p2);
+        if (f.type == RPX_FACE_DISTORTION) return distortion_intersect<F>(S, f, g);
     }
-    return plain_intersect<F>(S, f, p1, p2, is_base);
+    return plain_intersect<F>(S, f, g, is_base);
 }
 
 // DistortionFace.compute_normal_c (cfaces.pyx:2418-2431)
@@ -638,7 +598,7 @@ RPX_DEV V3 face_normal(const SceneView &S, const rpx_face_t &f, V3 p) {
     n.z = 1.0;
     n.x -= dxdyz.x;
     n.y -= dxdyz.y;
-    return norm(n);
+    return unit(n);
 }
 
 // compute_tangent_c: (1,0,0) by default, (0,0,1) for ExtrudedPlanarFace
@@ -656,7 +616,7 @@ struct Orientation {
 template <uint32_t F>
 RPX_DEV Orientation compute_orientation(const SceneView &S, const rpx_face_list_t &fl,
                                         const rpx_face_t &f, V3 point) {
-    point = transform(fl.inv_trans, point);
+    point = to_local(fl, point);
     Orientation o;
     o.normal = face_normal<F>(S, f, point);
     o.tangent = face_tangent(f);
@@ -664,9 +624,60 @@ RPX_DEV Orientation compute_orientation(const SceneView &S, const rpx_face_list_
         o.normal = neg(o.normal);
         o.tangent = neg(o.tangent);
     }
-    o.normal = rotate(fl.trans, o.normal);
-    o.tangent = rotate(fl.trans, o.tangent);
+    o.normal = to_global_dir(fl, o.normal);
+    o.tangent = to_global_dir(fl, o.tangent);
     return o;
+}
+
+// ---------------------------------------------------------- nearest face
+struct NearHit {
+    double length;
+    uint32_t end_face;
+    int rec, list;          // face record and face list, -1 without a hit
+};
+
+// trace_segment_c / FaceList.intersect_c (ctracer.pyx:2093-2104, 1882-1904), or
+// with one_list >= 0 FaceList.intersect_one_face_c (:1861-1879): the first of
+// the nearest faces closer than `length`.  Face lists whose frame is the
+// global one share one segment.  Face and list indices are the same in every
+// lane; with SCALAR the face records are read from `faces` in global memory by
+// scalar loads (into SGPRs), otherwise from the LDS copy S holds.
+template <uint32_t F, bool SCALAR>
+RPX_DEV NearHit nearest_face(const SceneView &S, const rpx_face_t *faces, V3 origin, V3 dir, double max_length,
+                             double length, int one_list, int one_face) {
+    NearHit h{length, RPX_NO_FACE, -1, -1};
+    const V3 point = add(origin, mul(dir, max_length));
+    const int l0 = one_list < 0 ? 0 : one_list, l1 = one_list < 0 ? S.n_face_lists : one_list + 1;
+    Seg g;
+    bool global_frame = false;   // g is in the global frame
+    for (int l = l0; l < l1; ++l) {
+        const rpx_face_list_t &fl = S.face_lists[l];
+        const int flags = __builtin_amdgcn_readfirstlane(fl.pad[0]);
+        if (flags & FL_INV_IDENTITY) {
+            if (!global_frame) g = make_seg(origin, point);
+            global_frame = true;
+        } else {
+            g = make_seg(transform(fl.inv_trans, origin), transform(fl.inv_trans, point));
+            global_frame = false;
+        }
+        const int k0 = __builtin_amdgcn_readfirstlane(one_list < 0 ? fl.first_face : fl.first_face + one_face);
+        const int k1 = __builtin_amdgcn_readfirstlane(one_list < 0 ? fl.first_face + fl.n_faces : k0 + 1);
+        for (int k = k0; k < k1; ++k) {
+            auto test = [&](const rpx_face_t &fc) {
+                if (face_out_of_reach(fc, g.p1.z, g.u.z * h.length, g.slen)) return;
+                const double dist = face_intersect<F>(S, fc, g, 1);
+                if (fc.tolerance < dist && dist < h.length) {
+                    h.length = dist;
+                    h.end_face = (uint32_t)fc.global_idx;
+                    h.rec = k;
+                    h.list = l;
+                }
+            };
+            if constexpr (SCALAR) test(face_uniform(faces, k));
+            else test(S.faces[k]);
+        }
+    }
+    return h;
 }
 
 }  // namespace rpx

@@ -20,21 +20,62 @@ struct Ray {
 // emitter does not take (a multi-order grating's third order, built again
 // after the children's positions are known).
 //
-// PairEmit collects the (at most two) children of one ray as a two-slot
-// shift register: r0 is the latest child, r1 the one before.  Conditional
-// or indexed slot writes make the compiler keep the pair in scratch memory;
-// the unconditional shift keeps both in registers.
+// PairEmit collects the (at most two) children of one ray: what a material
+// gives both of them alike once (hit point, normal, polarisation basis,
+// lengths, wavelength, identity), and direction, index, amplitudes, phase and
+// type per child in a two-slot shift register (s0 is the latest child, s1 the
+// one before).  Conditional or indexed slot writes make the compiler keep the
+// pair in scratch memory; the unconditional shift keeps both in registers,
+// 66 of them where two whole records took 94.
 struct PairEmit {
     static constexpr int kCap = 2;
-    Ray r0, r1;
+    struct Slot {
+        V3 direction;
+        Cx n, E1, E2;
+        double phase;
+        uint32_t type;
+    };
+    V3 origin, normal, E_vector;
+    double length, accum;
+    uint32_t wl_idx, parent_idx, end_face_idx, ray_ident;
+    Slot s0, s1;
     int n = 0;
     RPX_DEV void operator()(const Ray &x) {
-        r1 = r0;
-        r0 = x;
+        origin = x.origin;
+        normal = x.normal;
+        E_vector = x.E_vector;
+        length = x.length;
+        accum = x.accum;
+        wl_idx = x.wl_idx;
+        parent_idx = x.parent_idx;
+        end_face_idx = x.end_face_idx;
+        ray_ident = x.ray_ident;
+        s1 = s0;
+        s0 = Slot{x.direction, x.n, x.E1, x.E2, x.phase, x.ray_type_id};
         ++n;
     }
     RPX_DEV void skip() { ++n; }
-    RPX_DEV const Ray &first() const { return n > 1 ? r1 : r0; }
+    RPX_DEV Ray child(const Slot &s) const {
+        Ray r;
+        r.origin = origin;
+        r.direction = s.direction;
+        r.normal = normal;
+        r.E_vector = E_vector;
+        r.n = s.n;
+        r.E1 = s.E1;
+        r.E2 = s.E2;
+        r.length = length;
+        r.phase = s.phase;
+        r.accum = accum;
+        r.wl_idx = wl_idx;
+        r.parent_idx = parent_idx;
+        r.end_face_idx = end_face_idx;
+        r.ray_ident = ray_ident;
+        r.ray_type_id = s.type;
+        return r;
+    }
+    RPX_DEV Ray first() const { return child(n > 1 ? s1 : s0); }
+    RPX_DEV Ray second() const { return child(s0); }
 };
 
 // Order k (0-based) of a grating: `order`, then the signed bytes of
@@ -132,26 +173,21 @@ RPX_DEV Cx eval_dispersion(const rpx_dispersion_t &d, double wvl) {
 }
 
 // ------------------------------------------------------------- S/P basis
-// convert_to_sp (cmaterials.pyx:49-91)
+// convert_to_sp (cmaterials.pyx:49-91) for a unit normal (which the
+// reference normalises once more).
 RPX_DEV Ray convert_to_sp(Ray ray, V3 normal) {
-    Cx E1 = ray.E1, E2 = ray.E2;
-    V3 E2v = norm(cross(ray.direction, ray.E_vector));
-    V3 E1v = norm(cross(E2v, ray.direction));
-    normal = norm(normal);
-    V3 S = cross(ray.direction, normal);
-    if (fabs(S.x) < 1.0e-10 && fabs(S.y) < 1.0e-10 && fabs(S.z) < 1.0e-10) return ray;
-    S = norm(S);
-    V3 v = cross(ray.direction, S);
-    V3 P = norm(v);
-    double A = dot(E1v, S);
-    double B = dot(E2v, S);
-    Cx Samp = cx(E1.re * A + E2.re * B, E1.im * A + E2.im * B);
+    const V3 S0 = cross(ray.direction, normal);
+    if (fabs(S0.x) < 1.0e-10 && fabs(S0.y) < 1.0e-10 && fabs(S0.z) < 1.0e-10) return ray;
+    const Cx E1 = ray.E1, E2 = ray.E2;
+    const V3 E2v = unit(cross(ray.direction, ray.E_vector));
+    const V3 E1v = unit(cross(E2v, ray.direction));
+    const V3 S = unit(S0), P = unit(cross(ray.direction, S));
+    double A = dot(E1v, S), B = dot(E2v, S);
+    ray.E1 = cx(E1.re * A + E2.re * B, E1.im * A + E2.im * B);
     B = dot(E1v, P);
     A = dot(E2v, P);
-    Cx Pamp = cx(E1.re * B + E2.re * A, E1.im * B + E2.im * A);
+    ray.E2 = cx(E1.re * B + E2.re * A, E1.im * B + E2.im * A);
     ray.E_vector = S;
-    ray.E1 = Samp;
-    ray.E2 = Pamp;
     return ray;
 }
 
@@ -191,9 +227,94 @@ RPX_DEV bool material_emits(const rpx_material_t &m) {
     return m.type != RPX_MAT_NONE && m.type != RPX_MAT_OPAQUE;
 }
 
-RPX_DEV double power_frac(double nre, Cx a, Cx b, double P_in) {
-    double ca = cabs_(a), cb = cabs_(b);
-    return nre * (ca * ca + cb * cb) / P_in;
+// |a|^2
+RPX_DEV double cnorm2(Cx a) { return fma(a.re, a.re, a.im * a.im); }
+
+// Amplitude coefficients of an interface: reflected and transmitted, s and p;
+// the transmitted ones carry sqrt(cos3 / cos1).
+struct Coefs {
+    Cx rs, rp, ts, tp;
+};
+
+// Bare interface n1 -> n2 (cmaterials.pyx:790-850).  Two real indices below
+// total reflection (`real`): cos2 is the transmitted ray's own cosine, and each
+// polarisation's pair shares one reciprocal.
+RPX_DEV Coefs fresnel_coefs(Cx n1, Cx n2, double cos1, double sin1, bool real, double cos2r) {
+    Coefs c;
+    if (real) {
+        const double n2c1 = n2.re * cos1, n1c2 = n1.re * cos2r, n2c2 = n2.re * cos2r, n1c1 = n1.re * cos1;
+        const double ip = 1.0 / (n2c1 + n1c2), is = 1.0 / (n2c2 + n1c1);
+        const double t = 2.0 * n1.re * sqrt(cos1 * cos2r);
+        c.rp = cx((n1c2 - n2c1) * ip, 0.0);
+        c.rs = cx((n1c1 - n2c2) * is, 0.0);
+        c.tp = cx(t * ip, 0.0);
+        c.ts = cx(t * is, 0.0);
+        return c;
+    }
+    const Cx sin2 = cdiv(cmul(n1, cx(sin1, 0.0)), n2);
+    const Cx cos2 = csqrt_(csub(cx(1, 0), cmul(sin2, sin2)));
+    const Cx n2c1 = cmul(n2, cx(cos1, 0)), n1c2 = cmul(n1, cos2);
+    const Cx n2c2 = cmul(n2, cos2), n1c1 = cmul(n1, cx(cos1, 0));
+    c.rp = cdiv(csub(n1c2, n2c1), cadd(n2c1, n1c2));
+    c.rs = cdiv(csub(n1c1, n2c2), cadd(n2c2, n1c1));
+    const double aspect = sqrt(cos2.re / cos1);
+    const Cx num = cmul(cx(aspect, 0), cmul(cx(2.0 * cos1, 0), n1));
+    c.tp = cdiv(num, cadd(n2c1, n1c2));
+    c.ts = cdiv(num, cadd(n2c2, n1c1));
+    return c;
+}
+
+// Interface n1 -> n3 under a film of index n2 (cmaterials.pyx:1026-1182,
+// 1228-1391).  With the reference's phi = -i dwc (n2 - sin2^2) / cos2 and, for
+// s, a, b = n1 cos1 -+ n2 cos2, c, d = n2 cos2 +- n3 cos3 (for p with the
+// cosines of the other side), its matrix elements M00 .. M11 give
+//   r = (a c + b d e^-2phi) / (a d e^-2phi + b c),
+//   t = M10 + M11 r = -(a^2 - b^2)(c^2 - d^2) e^-phi / (4 n2 cos2 n3 cos3 (..)),
+// and a^2 - b^2 is a product again: 4 n1 cos1 n2 cos2 e^-phi over the same
+// denominator for s, 4 n1 cos2 n2 cos1 e^-phi for p.  Three real indices below
+// total reflection (`real`): e^phi has modulus 1 and the rest is real.
+RPX_DEV Coefs film_coefs(Cx n1, Cx n2, Cx n3, double cos1, double sin1, double dwc, bool real, double sin1sq,
+                         double cos3r) {
+    Coefs o;
+    if (real) {
+        const double q = n1.re / n2.re, sin2sq = sin1sq * q * q;
+        const double cos2 = sqrt(1.0 - sin2sq);
+        double sp, cp;   // e^-phi = cp + i sp
+        sincos(dwc * (n2.re - sin2sq) / cos2, &sp, &cp);
+        const double er = fma(cp, cp, -(sp * sp)), ei = 2.0 * sp * cp;   // e^-2phi
+        const double n1c1 = n1.re * cos1, n2c2 = n2.re * cos2, n3c3 = n3.re * cos3r;
+        const double n1c2 = n1.re * cos2, n2c1 = n2.re * cos1, n2c3 = n2.re * cos3r, n3c2 = n3.re * cos2;
+        const double aspect = 4.0 * sqrt(cos3r / cos1);
+        auto pol = [&](double a, double b, double c, double d, double t, Cx &r_out, Cx &t_out) {
+            const double ac = a * c, bd = b * d, ad = a * d, bc = b * c;
+            const double dr = fma(ad, er, bc), di = ad * ei;
+            const double nr = fma(bd, er, ac), ni = bd * ei;
+            const double inv = 1.0 / fma(dr, dr, di * di);
+            r_out = cx(fma(nr, dr, ni * di) * inv, fma(ni, dr, -(nr * di)) * inv);
+            t *= aspect * inv;
+            t_out = cx(fma(cp, dr, sp * di) * t, fma(sp, dr, -(cp * di)) * t);
+        };
+        pol(n1c1 - n2c2, n1c1 + n2c2, n2c2 + n3c3, n2c2 - n3c3, n1c1 * n2c2, o.rs, o.ts);
+        pol(n1c2 - n2c1, n1c2 + n2c1, n2c3 + n3c2, n2c3 - n3c2, n1c2 * n2c1, o.rp, o.tp);
+        return o;
+    }
+    const Cx n1s1 = cmul(n1, cx(sin1, 0));
+    const Cx sin2 = cdiv(n1s1, n2), sin3 = cdiv(n1s1, n3);
+    const Cx s2 = cmul(sin2, sin2);
+    const Cx cos2 = csqrt_(csub(cx(1, 0), s2)), cos3 = csqrt_(csub(cx(1, 0), cmul(sin3, sin3)));
+    const Cx mphi = cdiv(cmul(cx(0.0, dwc), csub(n2, s2)), cos2);    // -phi
+    const Cx e1 = cexp_(mphi), e2 = cexp_(cmul(cx(2, 0), mphi));
+    const Cx n1c1 = cmul(n1, cx(cos1, 0)), n2c2 = cmul(n2, cos2), n3c3 = cmul(n3, cos3);
+    const Cx n1c2 = cmul(n1, cos2), n2c1 = cmul(n2, cx(cos1, 0)), n2c3 = cmul(n2, cos3), n3c2 = cmul(n3, cos2);
+    const double aspect = 4.0 * sqrt(cos3.re / cos1);
+    auto pol = [&](Cx a, Cx b, Cx c, Cx d, Cx t, Cx &r_out, Cx &t_out) {
+        const Cx den = cadd(cmul(cmul(a, d), e2), cmul(b, c));
+        r_out = cdiv(cadd(cmul(a, c), cmul(cmul(b, d), e2)), den);
+        t_out = cdiv(cmul(cmul(t, cx(aspect, 0)), e1), den);
+    };
+    pol(csub(n1c1, n2c2), cadd(n1c1, n2c2), cadd(n2c2, n3c3), csub(n2c2, n3c3), cmul(n1c1, n2c2), o.rs, o.ts);
+    pol(csub(n1c2, n2c1), cadd(n1c2, n2c1), cadd(n2c3, n3c2), csub(n2c3, n3c2), cmul(n1c2, n2c1), o.rp, o.tp);
+    return o;
 }
 
 // ------------------------------------------------------------- children
@@ -204,12 +325,12 @@ RPX_DEV double power_frac(double nre, Cx a, Cx b, double P_in) {
 template <class Emit>
 RPX_DEV void grating_children(const rpx_material_t &m, const Ray &in, uint32_t idx, V3 point,
                               const Orientation &orient, const WlTable &wavelengths, Emit &emit) {
-    V3 normal = norm(orient.normal);
-    V3 tangent = norm(orient.tangent);
+    V3 normal = unit(orient.normal);
+    V3 tangent = unit(orient.tangent);
     V3 tangent2 = cross(normal, tangent);
     double wavelen = wavelengths[in.wl_idx];
     double line_spacing = 1000.0 / m.lines_per_mm;
-    const V3 dir = norm(in.direction);
+    const V3 dir = unit(in.direction);
     const double k_z0 = dot(normal, dir);
     const double k_y = dot(tangent2, dir);
     const double k_x0 = dot(tangent, dir);
@@ -254,7 +375,7 @@ RPX_DEV void eval_children(const rpx_material_t &m, const Ray &in, uint32_t idx,
     switch (m.type) {
     case RPX_MAT_TRANSPARENT: {
         if constexpr ((F & M_SIMPLE) == 0) return;  // cmaterials.pyx:260-278
-        V3 normal = norm(orient.normal);
+        V3 normal = unit(orient.normal);
         Ray sp = convert_to_sp(in, normal);
         sp.accum += sp.length * sp.n.re;
         sp.origin = point;
@@ -266,7 +387,7 @@ RPX_DEV void eval_children(const rpx_material_t &m, const Ray &in, uint32_t idx,
     } break;
     case RPX_MAT_PEC: {
         if constexpr ((F & M_SIMPLE) == 0) return;  // cmaterials.pyx:285-319
-        V3 normal = norm(orient.normal);
+        V3 normal = unit(orient.normal);
         Ray sp = convert_to_sp(in, normal);
         double cosTheta = dot(normal, in.direction);
         V3 ctn = mul(normal, cosTheta);
@@ -284,8 +405,8 @@ RPX_DEV void eval_children(const rpx_material_t &m, const Ray &in, uint32_t idx,
     } break;
     case RPX_MAT_PARTIAL: {
         if constexpr ((F & M_SIMPLE) == 0) return;  // cmaterials.pyx:345-397
-        V3 normal = norm(orient.normal);
-        V3 in_dir = norm(in.direction);
+        V3 normal = unit(orient.normal);
+        V3 in_dir = unit(in.direction);
         Ray sp = convert_to_sp(in, normal);
         double cosTheta = dot(normal, in_dir);
         V3 ctn = mul(normal, cosTheta);
@@ -315,8 +436,8 @@ RPX_DEV void eval_children(const rpx_material_t &m, const Ray &in, uint32_t idx,
     } break;
     case RPX_MAT_DIELECTRIC: {
         if constexpr ((F & M_SIMPLE) == 0) return;  // cmaterials.pyx:587-680
-        V3 normal = norm(orient.normal);
-        V3 in_dir = norm(in.direction);
+        V3 normal = unit(orient.normal);
+        V3 in_dir = unit(in.direction);
         Ray sp = convert_to_sp(in, normal);
         sp.accum += sp.length * sp.n.re;
         double cosTheta = dot(normal, in_dir);
@@ -371,155 +492,68 @@ RPX_DEV void eval_children(const rpx_material_t &m, const Ray &in, uint32_t idx,
         emit(sp);
     } break;
     case RPX_MAT_FULL_DIELECTRIC:
-    case RPX_MAT_FULL_DISPERSIVE: {
-        if constexpr ((F & M_FRESNEL) == 0) return;  // cmaterials.pyx:755-872, 896-1013
-        Sides sd = material_indices(m, m.type == RPX_MAT_FULL_DISPERSIVE ? wavelengths[in.wl_idx] : 0.0);
-        V3 normal = norm(orient.normal);
-        V3 in_dir = norm(in.direction);
-        Ray sp = convert_to_sp(in, normal);
-        sp.accum += sp.length * sp.n.re;
-        Cx E1 = sp.E1, E2 = sp.E2;
-        double cosTheta = dot(normal, in_dir);
-        double cos1 = fabs(cosTheta);
-        double sin1 = sqrt(fabs(1 - cos1 * cos1));
-        Cx n1, n2;
-        int flip;
-        if (cosTheta < 0.0) { n1 = sd.n_out; n2 = sd.n_in; flip = 1; }
-        else { n1 = sd.n_in; n2 = sd.n_out; flip = -1; }
-        Cx sin2 = cdiv(cmul(n1, R(sin1)), n2);
-        Cx cos2 = csqrt_(csub(R(1), cmul(sin2, sin2)));
-        V3 ctn = mul(normal, cosTheta);
-        double P_in = n1.re * (E1.re * E1.re + E1.im * E1.im + E2.re * E2.re + E2.im * E2.im);
-        if (P_in == 0.0) return;
-        Cx n2c1 = cmul(n2, R(cos1)), n1c2 = cmul(n1, cos2);
-        Cx n2c2 = cmul(n2, cos2), n1c1 = cmul(n1, R(cos1));
-        Cx R_p = cdiv(cneg(csub(n2c1, n1c2)), cadd(n2c1, n1c2));
-        Cx R_s = cdiv(cneg(csub(n2c2, n1c1)), cadd(n2c2, n1c1));
-        R_s = cmul(R_s, E1);
-        R_p = cmul(R_p, E2);
-        if (power_frac(n1.re, R_s, R_p, P_in) > m.reflection_threshold) {
-            Ray c = sp;
-            c.origin = point;
-            c.normal = normal;
-            c.direction = sub(in_dir, mul(ctn, 2));
-            c.length = RPX_INF;
-            c.E1 = R_s;
-            c.E2 = cx(-R_p.re, -R_p.im);
-            c.parent_idx = idx;
-            c.n = n1;
-            c.ray_type_id |= RPX_REFL_RAY;
-            emit(c);
-            sp = c;
-        }
-        V3 tangent = sub(in_dir, ctn);
-        V3 tg2 = mul(tangent, n1.re / n2.re);
-        double tan_mag_sq = mag_sq(tg2);
-        double c2 = sqrt(1 - tan_mag_sq);
-        V3 transmitted = sub(tg2, mul(normal, c2 * flip));
-        double aspect = sqrt(cos2.re / cos1);
-        Cx num = cmul(R(aspect), cmul(R(2.0 * cos1), n1));
-        Cx T_p = cdiv(num, cadd(n2c1, n1c2));
-        Cx T_s = cdiv(num, cadd(n2c2, n1c1));
-        T_s = cmul(T_s, E1);
-        T_p = cmul(T_p, E2);
-        if (power_frac(n2.re, T_s, T_p, P_in) > m.transmission_threshold) {
-            sp.origin = point;
-            sp.normal = normal;
-            sp.direction = transmitted;
-            sp.length = RPX_INF;
-            sp.E1 = T_s;
-            sp.E2 = T_p;
-            sp.parent_idx = idx;
-            sp.n = n2;
-            sp.ray_type_id &= ~RPX_REFL_RAY;
-            emit(sp);
-        }
-    } break;
+    case RPX_MAT_FULL_DISPERSIVE:
     case RPX_MAT_SINGLE_LAYER:
     case RPX_MAT_COATED_DISPERSIVE: {
-        if constexpr ((F & M_COATED) == 0) return;  // cmaterials.pyx:1026-1182, 1228-1391
-        const double wavelength = wavelengths[in.wl_idx];  // both read _wavelengths
-        Sides sd = material_indices(m, wavelength);
-        V3 normal = norm(orient.normal);
-        V3 in_dir = norm(in.direction);
+        // FullDielectricMaterial and its dispersive form (cmaterials.pyx:755-872,
+        // 896-1013), SingleLayerCoated and CoatedDispersive (:1026-1182, 1228-1391)
+        if constexpr ((F & (M_FRESNEL | M_COATED)) == 0) return;
+        const bool film = m.type == RPX_MAT_SINGLE_LAYER || m.type == RPX_MAT_COATED_DISPERSIVE;
+        const double wavelength = m.type == RPX_MAT_FULL_DIELECTRIC ? 0.0 : wavelengths[in.wl_idx];
+        const Sides sd = material_indices(m, wavelength);
+        V3 normal = unit(orient.normal);
+        V3 in_dir = unit(in.direction);
         Ray sp = convert_to_sp(in, normal);
         sp.accum += sp.length * sp.n.re;
-        Cx E1 = sp.E1, E2 = sp.E2;
-        double cosTheta = dot(normal, in_dir);
-        double cos1 = fabs(cosTheta);
-        double sin1 = sqrt(fabs(1 - cos1 * cos1));
-        Cx n2 = sd.n_coat, n1, n3;
-        int flip;
-        if (cosTheta < 0.0) { n1 = sd.n_out; n3 = sd.n_in; flip = 1; }
-        else { n1 = sd.n_in; n3 = sd.n_out; flip = -1; }
-        Cx n1s1 = cmul(n1, R(sin1));
-        Cx sin2 = cdiv(n1s1, n2);
-        Cx cos2 = csqrt_(csub(R(1), cmul(sin2, sin2)));
-        Cx sin3 = cdiv(n1s1, n3);
-        Cx cos3 = csqrt_(csub(R(1), cmul(sin3, sin3)));
-        V3 ctn = mul(normal, cosTheta);
-        double P_in = n1.re * (E1.re * E1.re + E1.im * E1.im + E2.re * E2.re + E2.im * E2.im);
+        sp.origin = point;
+        sp.normal = normal;
+        sp.length = RPX_INF;
+        sp.parent_idx = idx;
+        const Cx E1 = sp.E1, E2 = sp.E2;
+        const double cosTheta = dot(normal, in_dir);
+        const double cos1 = fabs(cosTheta);
+        const bool inward = cosTheta < 0.0;
+        const Cx n1 = inward ? sd.n_out : sd.n_in, n3 = inward ? sd.n_in : sd.n_out;
+        const double P_in = n1.re * (cnorm2(E1) + cnorm2(E2));
         if (P_in == 0.0) return;
-        Cx n1cos1 = cmul(n1, R(cos1));
-        Cx n2cos2 = cmul(n2, cos2);
-        Cx n3cos3 = cmul(n3, cos3);
-        double dwc = 2 * M_PI * m.thickness / wavelength;
-        Cx phi = cdiv(cmul(cmul(cx(-0.0, -1.0), R(dwc)), csub(n2, cmul(sin2, sin2))), cos2);
-        Cx ep1 = cdiv(cexp_(phi), cmul(cmul(R(4), n2cos2), n3cos3));
-        Cx ep2 = cexp_(cmul(R(-2), phi));
-        Cx mep1 = cneg(ep1);
-        // s-polarisation
-        Cx a = csub(n1cos1, n2cos2), b = cadd(n1cos1, n2cos2);
-        Cx c = cadd(n2cos2, n3cos3), d = csub(n2cos2, n3cos3);
-        Cx M00 = cmul(mep1, cadd(cmul(a, c), cmul(cmul(b, d), ep2)));
-        Cx M01 = cmul(ep1, cadd(cmul(cmul(a, d), ep2), cmul(b, c)));
-        Cx M10 = cmul(ep1, cadd(cmul(a, d), cmul(cmul(b, c), ep2)));
-        Cx M11 = cmul(mep1, cadd(cmul(cmul(a, c), ep2), cmul(b, d)));
-        Cx R_s = cdiv(cneg(M00), M01);
-        Cx T_s = cadd(M10, cmul(M11, R_s));
-        // p-polarisation
-        Cx n1cos2 = cmul(n1, cos2), n2cos1 = cmul(n2, R(cos1));
-        Cx n2cos3 = cmul(n2, cos3), n3cos2 = cmul(n3, cos2);
-        a = csub(n1cos2, n2cos1); b = cadd(n1cos2, n2cos1);
-        c = cadd(n2cos3, n3cos2); d = csub(n2cos3, n3cos2);
-        M00 = cmul(mep1, cadd(cmul(a, c), cmul(cmul(b, d), ep2)));
-        M01 = cmul(ep1, cadd(cmul(cmul(a, d), ep2), cmul(b, c)));
-        M10 = cmul(ep1, cadd(cmul(a, d), cmul(cmul(b, c), ep2)));
-        M11 = cmul(mep1, cadd(cmul(cmul(a, c), ep2), cmul(b, d)));
-        Cx R_p = cdiv(cneg(M00), M01);
-        Cx T_p = cadd(M10, cmul(M11, R_p));
-        R_s = cmul(R_s, E1);
-        R_p = cmul(R_p, E2);
-        if (power_frac(n1.re, R_s, R_p, P_in) > m.reflection_threshold) {
-            Ray cr = sp;
-            cr.origin = point;
-            cr.normal = normal;
-            cr.direction = sub(in_dir, mul(ctn, 2));
-            cr.length = RPX_INF;
-            cr.E1 = R_s;
-            cr.E2 = cx(-R_p.re, -R_p.im);
-            cr.parent_idx = idx;
-            cr.n = n1;
-            cr.ray_type_id |= RPX_REFL_RAY;
-            emit(cr);
-            sp = cr;
+        const double per_P = 1.0 / P_in;
+        // the tangential part of the direction, before and after refraction
+        const V3 tangent = sub(in_dir, mul(normal, cosTheta));
+        const V3 tg2 = mul(tangent, n1.re / n3.re);
+        const double tan_mag_sq = mag_sq(tg2);
+        const double c2 = sqrt(1 - tan_mag_sq);
+        bool real = n1.im == 0.0 && n3.im == 0.0 && n1.re > 0.0 && n3.re > 0.0 && tan_mag_sq < 1.0;
+        Coefs k;
+        if (film) {
+            if constexpr ((F & M_COATED) != 0) {
+                const double sin1sq = mag_sq(tangent);
+                real = real && sd.n_coat.im == 0.0 && sd.n_coat.re > 0.0 &&
+                       n1.re * n1.re * sin1sq < sd.n_coat.re * sd.n_coat.re;
+                k = film_coefs(n1, sd.n_coat, n3, cos1, sqrt(fabs(1 - cos1 * cos1)),
+                               2 * M_PI * m.thickness / wavelength, real, sin1sq, c2);
+            } else {
+                return;
+            }
+        } else {
+            if constexpr ((F & M_FRESNEL) != 0)
+                k = fresnel_coefs(n1, n3, cos1, sqrt(fabs(1 - cos1 * cos1)), real, c2);
+            else
+                return;
         }
-        V3 tangent = sub(in_dir, ctn);
-        V3 tg2 = mul(tangent, n1.re / n3.re);
-        double tan_mag_sq = mag_sq(tg2);
-        double c2 = sqrt(1 - tan_mag_sq);
-        V3 transmitted = sub(tg2, mul(normal, c2 * flip));
-        double aspect = sqrt(cos3.re / cos1);
-        T_s = cmul(T_s, cmul(E1, R(aspect)));
-        T_p = cmul(T_p, cmul(E2, R(aspect)));
-        if (power_frac(n3.re, T_s, T_p, P_in) > m.transmission_threshold) {
-            sp.origin = point;
-            sp.normal = normal;
-            sp.direction = transmitted;
-            sp.length = RPX_INF;
+        const Cx R_s = cmul(k.rs, E1), R_p = cmul(k.rp, E2);
+        if (n1.re * (cnorm2(R_s) + cnorm2(R_p)) * per_P > m.reflection_threshold) {
+            sp.direction = sub(in_dir, mul(mul(normal, cosTheta), 2));
+            sp.E1 = R_s;
+            sp.E2 = cx(-R_p.re, -R_p.im);
+            sp.n = n1;
+            sp.ray_type_id |= RPX_REFL_RAY;
+            emit(sp);
+        }
+        const Cx T_s = cmul(k.ts, E1), T_p = cmul(k.tp, E2);
+        if (n3.re * (cnorm2(T_s) + cnorm2(T_p)) * per_P > m.transmission_threshold) {
+            sp.direction = sub(tg2, mul(normal, inward ? c2 : -c2));
             sp.E1 = T_s;
             sp.E2 = T_p;
-            sp.parent_idx = idx;
             sp.n = n3;
             sp.ray_type_id &= ~RPX_REFL_RAY;
             emit(sp);
@@ -541,14 +575,14 @@ template <uint32_t F>
 RPX_DEV Para eval_parabasal(const rpx_material_t &m, const Ray &base, V3 direction, V3 point,
                             const Orientation &orient, uint32_t ray_type_id, const WlTable &wavelengths) {
     Para out;
-    V3 normal = norm(orient.normal);
+    V3 normal = unit(orient.normal);
     switch (m.type) {
     case RPX_MAT_DIELECTRIC:
     case RPX_MAT_FULL_DIELECTRIC:
     case RPX_MAT_SINGLE_LAYER:
     case RPX_MAT_COATED_DISPERSIVE: {
         if constexpr ((F & (M_SIMPLE | M_FRESNEL | M_COATED)) == 0) break;
-        direction = norm(direction);
+        direction = unit(direction);
         double cosTheta = dot(normal, direction);
         V3 ctn = mul(normal, cosTheta);
         double n1, n2;
@@ -576,11 +610,11 @@ RPX_DEV Para eval_parabasal(const rpx_material_t &m, const Ray &base, V3 directi
     } break;
     case RPX_MAT_GRATING: {
         if constexpr ((F & M_GRATING) == 0) break;
-        V3 tangent = norm(orient.tangent);
+        V3 tangent = unit(orient.tangent);
         V3 tangent2 = cross(normal, tangent);
         double wavelen = wavelengths[base.wl_idx];
         double line_spacing = 1000.0 / m.lines_per_mm;
-        V3 reflected = norm(direction);
+        V3 reflected = unit(direction);
         double k_z = dot(normal, reflected);
         double k_y = dot(tangent2, reflected);
         double k_x = dot(tangent, reflected);

@@ -3,6 +3,7 @@
 // InterfaceMaterial.eval_child_ray of the Python API.
 #include <hip/hip_runtime.h>
 #include "rpx_materials.h"
+#include "rpx_faces_ref.h"
 #include "rpx_host.h"
 
 using namespace rpx;
@@ -15,7 +16,7 @@ __global__ void k_query_face(SceneView S, int rec, int what, const double *p1, c
     V3 a = v3(p1[3 * i], p1[3 * i + 1], p1[3 * i + 2]);
     if (what == 0) {
         V3 b = v3(p2[3 * i], p2[3 * i + 1], p2[3 * i + 2]);
-        out[i] = face_intersect<V_ALL>(S, f, a, b, is_base);
+        out[i] = ref::face_intersect<V_ALL>(S, f, a, b, is_base);
     } else {
         V3 nrm = face_normal<V_ALL>(S, f, a);
         out[3 * i] = nrm.x;

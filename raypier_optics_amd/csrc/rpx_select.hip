@@ -13,6 +13,7 @@
 #include <algorithm>
 #include <string>
 #include "rpx_materials.h"
+#include "rpx_faces_ref.h"
 #include "rpx_host.h"
 #include "rpx_gen.h"
 
@@ -56,7 +57,7 @@ __global__ __launch_bounds__(RPX_BLOCK) void k_select(SelectArgs A) {
         const V3 p2 = transform(fl.inv_trans, point);
         for (int k = fl.first_face; k < fl.first_face + fl.n_faces; ++k) {
             const rpx_face_t &fc = S.faces[k];
-            const double dist = face_intersect<F>(S, fc, p1, p2, 1);
+            const double dist = ref::face_intersect<F>(S, fc, p1, p2, 1);
             if (fc.tolerance < dist && dist < length) {
                 length = dist;
                 end_face = (uint32_t)fc.global_idx;

@@ -158,7 +158,7 @@ __global__ __launch_bounds__(256) void k_batch_relayout(BatchJob *jobs, BatchCon
 }
 
 template <uint32_t F>
-__global__ __launch_bounds__(RPX_BLOCK) __attribute__((amdgpu_waves_per_eu(F == V_ALL ? 1 : 3)))
+__global__ __launch_bounds__(RPX_BLOCK) __attribute__((amdgpu_waves_per_eu(F == V_ALL ? 3 : 4)))
 void k_batch(const BatchJob *jobs, BatchControl *ctl, uint64_t *status,
                                                      double *partials) {
     __shared__ SceneLds lds_scene;
@@ -203,28 +203,10 @@ void k_batch(const BatchJob *jobs, BatchControl *ctl, uint64_t *status,
             const uint64_t c = J.in.capacity;
             const V3 origin = v3(f[RPX_OX * c + i], f[RPX_OY * c + i], f[RPX_OZ * c + i]);
             const V3 dir = v3(f[RPX_DX * c + i], f[RPX_DY * c + i], f[RPX_DZ * c + i]);
-            double length = J.max_length;
-            uint32_t end_face = RPX_NO_FACE;
-            int hit_rec = -1, hit_list = -1;
-            const V3 point = add(origin, mul(dir, J.max_length));
-            // trace_segment_c / FaceList.intersect_c (ctracer.pyx:2093-2104, 1882-1904)
-            for (int l = 0; l < S.n_face_lists; ++l) {
-                const rpx_face_list_t &fl = S.face_lists[l];
-                const V3 p1 = transform(fl.inv_trans, origin);
-                const V3 p2 = transform(fl.inv_trans, point);
-                const double slen = sep(p1, p2), zrate = (p2.z - p1.z) / slen;
-                for (int k = fl.first_face; k < fl.first_face + fl.n_faces; ++k) {
-                    const rpx_face_t &fc = S.faces[k];
-                    if (face_out_of_reach(fc, p1.z, zrate * length, slen)) continue;
-                    const double dist = face_intersect<F>(S, fc, p1, p2, 1);
-                    if (fc.tolerance < dist && dist < length) {
-                        length = dist;
-                        end_face = (uint32_t)fc.global_idx;
-                        hit_rec = k;
-                        hit_list = l;
-                    }
-                }
-            }
+            const NearHit nh = nearest_face<F, F != V_ALL>(S, J.S.faces, origin, dir, J.max_length, J.max_length, -1, -1);
+            const double length = nh.length;
+            const uint32_t end_face = nh.end_face;
+            const int hit_rec = nh.rec, hit_list = nh.list;
             J.in.f64[RPX_LENGTH * c + i] = length;
             J.in.u32[RPX_END_FACE_IDX * c + i] = end_face;
             if (hit_rec >= 0) {
@@ -276,7 +258,7 @@ void k_batch(const BatchJob *jobs, BatchControl *ctl, uint64_t *status,
         __syncthreads();
         const uint64_t pos = lds_excl + local;
         if (count > 0 && pos < J.out.capacity) store_ray(J.out, pos, ce.first());
-        if (count > 1 && pos + 1 < J.out.capacity) store_ray(J.out, pos + 1, ce.r0);
+        if (count > 1 && pos + 1 < J.out.capacity) store_ray(J.out, pos + 1, ce.second());
         if (threadIdx.x == 0) {
             if (lds_hits) atomicAdd((unsigned long long *)&J.counts[1], (unsigned long long)lds_hits);
             if (lds_parents) atomicAdd((unsigned long long *)&J.counts[2], (unsigned long long)lds_parents);

@@ -145,8 +145,77 @@ RPX_DEV RayS convert_to_sp_s(RayS ray, F3 normal) {
     return ray;
 }
 
-RPX_DEV float power_frac_s(float nre, Cf a, Cf b, float P_in) {
-    return nre * (cfabs2(a) + cfabs2(b)) / P_in;
+// Amplitude coefficients of an interface (rpx_materials.h, Coefs) in float32.
+struct CoefsS {
+    Cf rs, rp, ts, tp;
+};
+
+RPX_DEV CoefsS fresnel_coefs_s(Cf n1, Cf n2, float cos1, float sin1, bool real, float cos2r) {
+    CoefsS c;
+    if (real) {
+        const float n2c1 = n2.re * cos1, n1c2 = n1.re * cos2r, n2c2 = n2.re * cos2r, n1c1 = n1.re * cos1;
+        const float ip = 1.0f / (n2c1 + n1c2), is = 1.0f / (n2c2 + n1c1);
+        const float t = 2.0f * n1.re * sqrtf(cos1 * cos2r);
+        c.rp = cf((n1c2 - n2c1) * ip, 0.0f);
+        c.rs = cf((n1c1 - n2c2) * is, 0.0f);
+        c.tp = cf(t * ip, 0.0f);
+        c.ts = cf(t * is, 0.0f);
+        return c;
+    }
+    const Cf sin2 = cfdiv(cfscale(n1, sin1), n2);
+    const Cf cos2 = cfsqrt(cfsub(cf(1, 0), cfmul(sin2, sin2)));
+    const Cf n2c1 = cfscale(n2, cos1), n1c2 = cfmul(n1, cos2);
+    const Cf n2c2 = cfmul(n2, cos2), n1c1 = cfscale(n1, cos1);
+    c.rp = cfdiv(cfsub(n1c2, n2c1), cfadd(n2c1, n1c2));
+    c.rs = cfdiv(cfsub(n1c1, n2c2), cfadd(n2c2, n1c1));
+    const Cf num = cfscale(n1, sqrtf(cos2.re / cos1) * 2.0f * cos1);
+    c.tp = cfdiv(num, cfadd(n2c1, n1c2));
+    c.ts = cfdiv(num, cfadd(n2c2, n1c1));
+    return c;
+}
+
+RPX_DEV CoefsS film_coefs_s(Cf n1, Cf n2, Cf n3, float cos1, float sin1, float dwc, bool real, float sin1sq,
+                            float cos3r) {
+    CoefsS o;
+    if (real) {
+        const float q = n1.re / n2.re, sin2sq = sin1sq * q * q;
+        const float cos2 = sqrtf(1.0f - sin2sq);
+        float sp, cp;
+        sincosf(dwc * (n2.re - sin2sq) / cos2, &sp, &cp);
+        const float er = cp * cp - sp * sp, ei = 2.0f * sp * cp;
+        const float n1c1 = n1.re * cos1, n2c2 = n2.re * cos2, n3c3 = n3.re * cos3r;
+        const float n1c2 = n1.re * cos2, n2c1 = n2.re * cos1, n2c3 = n2.re * cos3r, n3c2 = n3.re * cos2;
+        const float aspect = 4.0f * sqrtf(cos3r / cos1);
+        auto pol = [&](float a, float b, float c, float d, float t, Cf &r_out, Cf &t_out) {
+            const float ac = a * c, bd = b * d, ad = a * d, bc = b * c;
+            const float dr = ad * er + bc, di = ad * ei;
+            const float nr = bd * er + ac, ni = bd * ei;
+            const float inv = 1.0f / (dr * dr + di * di);
+            r_out = cf((nr * dr + ni * di) * inv, (ni * dr - nr * di) * inv);
+            t *= aspect * inv;
+            t_out = cf((cp * dr + sp * di) * t, (sp * dr - cp * di) * t);
+        };
+        pol(n1c1 - n2c2, n1c1 + n2c2, n2c2 + n3c3, n2c2 - n3c3, n1c1 * n2c2, o.rs, o.ts);
+        pol(n1c2 - n2c1, n1c2 + n2c1, n2c3 + n3c2, n2c3 - n3c2, n1c2 * n2c1, o.rp, o.tp);
+        return o;
+    }
+    const Cf n1s1 = cfscale(n1, sin1);
+    const Cf sin2 = cfdiv(n1s1, n2), sin3 = cfdiv(n1s1, n3);
+    const Cf s2 = cfmul(sin2, sin2);
+    const Cf cos2 = cfsqrt(cfsub(cf(1, 0), s2)), cos3 = cfsqrt(cfsub(cf(1, 0), cfmul(sin3, sin3)));
+    const Cf mphi = cfdiv(cfmul(cf(0.0f, dwc), cfsub(n2, s2)), cos2);
+    const Cf e1 = cfexp(mphi), e2 = cfexp(cfscale(mphi, 2.0f));
+    const Cf n1c1 = cfscale(n1, cos1), n2c2 = cfmul(n2, cos2), n3c3 = cfmul(n3, cos3);
+    const Cf n1c2 = cfmul(n1, cos2), n2c1 = cfscale(n2, cos1), n2c3 = cfmul(n2, cos3), n3c2 = cfmul(n3, cos2);
+    const float aspect = 4.0f * sqrtf(cos3.re / cos1);
+    auto pol = [&](Cf a, Cf b, Cf c, Cf d, Cf t, Cf &r_out, Cf &t_out) {
+        const Cf den = cfadd(cfmul(cfmul(a, d), e2), cfmul(b, c));
+        r_out = cfdiv(cfadd(cfmul(a, c), cfmul(cfmul(b, d), e2)), den);
+        t_out = cfdiv(cfmul(cfscale(t, aspect), e1), den);
+    };
+    pol(cfsub(n1c1, n2c2), cfadd(n1c1, n2c2), cfadd(n2c2, n3c3), cfsub(n2c2, n3c3), cfmul(n1c1, n2c2), o.rs, o.ts);
+    pol(cfsub(n1c2, n2c1), cfadd(n1c2, n2c1), cfadd(n2c3, n3c2), cfsub(n2c3, n3c2), cfmul(n1c2, n2c1), o.rp, o.tp);
+    return o;
 }
 
 // Float64 refraction of in_dir (unit) at unit normal with index ratio n1/n2
@@ -181,13 +250,13 @@ RPX_DEV RayS begin_child(const RayS &in, double length, F3 normal_f, V3 point, u
 template <class Emit>
 RPX_DEV void grating_children_split(const rpx_material_t &m, const RayS &in, double length, uint32_t idx, V3 point,
                                     const Orientation &orient, const WlTable &wavelengths, Emit &emit) {
-    const V3 normal = norm(orient.normal);
+    const V3 normal = unit(orient.normal);
     const F3 normal_f = f3_of(normal);
-    const V3 tangent = norm(orient.tangent);
+    const V3 tangent = unit(orient.tangent);
     const V3 tangent2 = cross(normal, tangent);
     const double wavelen = wavelengths[in.wl_idx];
     const double line_spacing = 1000.0 / m.lines_per_mm;
-    const V3 dir = norm(v3_of(in.direction));
+    const V3 dir = unit(v3_of(in.direction));
     const double k_z0 = dot(normal, dir);
     const double k_y = dot(tangent2, dir);
     const double k_x0 = dot(tangent, dir);
@@ -223,7 +292,7 @@ RPX_DEV void grating_children_split(const rpx_material_t &m, const RayS &in, dou
 template <uint32_t F, class Emit>
 RPX_DEV void eval_children_split(const rpx_material_t &m, const RayS &in, double length, uint32_t idx,
                                  V3 point, const Orientation &orient, const WlTable &wavelengths, Emit &emit) {
-    const V3 normal = norm(orient.normal);
+    const V3 normal = unit(orient.normal);
     const F3 normal_f = f3_of(normal);
     switch (m.type) {
     case RPX_MAT_TRANSPARENT: {
@@ -243,7 +312,7 @@ RPX_DEV void eval_children_split(const rpx_material_t &m, const RayS &in, double
     } break;
     case RPX_MAT_PARTIAL: {
         if constexpr ((F & M_SIMPLE) == 0) return;
-        V3 in_dir = norm(v3_of(in.direction));
+        V3 in_dir = unit(v3_of(in.direction));
         RayS sp = begin_child(in, length, normal_f, point, idx);
         RayS sp2 = sp;
         const float Rr = sqrtf((float)m.reflectivity), T = sqrtf((float)(1 - m.reflectivity));
@@ -260,7 +329,7 @@ RPX_DEV void eval_children_split(const rpx_material_t &m, const RayS &in, double
     } break;
     case RPX_MAT_DIELECTRIC: {
         if constexpr ((F & M_SIMPLE) == 0) return;
-        V3 in_dir = norm(v3_of(in.direction));
+        V3 in_dir = unit(v3_of(in.direction));
         RayS sp = begin_child(in, length, normal_f, point, idx);
         const double cosTheta = dot(normal, in_dir);
         const double cos1 = fabs(cosTheta);
@@ -296,125 +365,60 @@ RPX_DEV void eval_children_split(const rpx_material_t &m, const RayS &in, double
         emit(sp);
     } break;
     case RPX_MAT_FULL_DIELECTRIC:
-    case RPX_MAT_FULL_DISPERSIVE: {
-        if constexpr ((F & M_FRESNEL) == 0) return;
-        Sides sd = material_indices(m, m.type == RPX_MAT_FULL_DISPERSIVE ? wavelengths[in.wl_idx] : 0.0);
-        V3 in_dir = norm(v3_of(in.direction));
-        RayS sp = begin_child(in, length, normal_f, point, idx);
-        const Cf E1 = sp.E1, E2 = sp.E2;
-        const double cosTheta = dot(normal, in_dir);
-        const double cos1d = fabs(cosTheta);
-        const float cos1 = (float)cos1d;
-        const float sin1 = sqrtf((float)fabs(1 - cos1d * cos1d));
-        Cx n1d, n2d;
-        int flip;
-        if (cosTheta < 0.0) { n1d = sd.n_out; n2d = sd.n_in; flip = 1; }
-        else { n1d = sd.n_in; n2d = sd.n_out; flip = -1; }
-        const Cf n1 = cf_of(n1d), n2 = cf_of(n2d);
-        const Cf sin2 = cfdiv(cfscale(n1, sin1), n2);
-        const Cf cos2 = cfsqrt(cfsub(cf(1, 0), cfmul(sin2, sin2)));
-        const float P_in = n1.re * (cfabs2(E1) + cfabs2(E2));
-        if (P_in == 0.0f) return;
-        const Cf n2c1 = cfscale(n2, cos1), n1c2 = cfmul(n1, cos2);
-        const Cf n2c2 = cfmul(n2, cos2), n1c1 = cfscale(n1, cos1);
-        Cf R_p = cfdiv(cfneg(cfsub(n2c1, n1c2)), cfadd(n2c1, n1c2));
-        Cf R_s = cfdiv(cfneg(cfsub(n2c2, n1c1)), cfadd(n2c2, n1c1));
-        R_s = cfmul(R_s, E1);
-        R_p = cfmul(R_p, E2);
-        if (power_frac_s(n1.re, R_s, R_p, P_in) > (float)m.reflection_threshold) {
-            RayS c = sp;
-            c.direction = f3_of(reflect_dir(in_dir, normal, cosTheta));
-            c.E1 = R_s;
-            c.E2 = cfneg(R_p);
-            c.n = n1;
-            c.ray_type_id |= RPX_REFL_RAY;
-            emit(c);
-            sp = c;
-        }
-        const V3 t = refract_dir(in_dir, normal, cosTheta, n1d.re / n2d.re, flip);
-        const float aspect = sqrtf(cos2.re / cos1);
-        const Cf num = cfscale(n1, aspect * 2.0f * cos1);
-        Cf T_p = cfdiv(num, cfadd(n2c1, n1c2));
-        Cf T_s = cfdiv(num, cfadd(n2c2, n1c1));
-        T_s = cfmul(T_s, E1);
-        T_p = cfmul(T_p, E2);
-        if (power_frac_s(n2.re, T_s, T_p, P_in) > (float)m.transmission_threshold) {
-            sp.direction = f3_of(t);
-            sp.E1 = T_s;
-            sp.E2 = T_p;
-            sp.n = n2;
-            sp.ray_type_id &= ~RPX_REFL_RAY;
-            emit(sp);
-        }
-    } break;
+    case RPX_MAT_FULL_DISPERSIVE:
     case RPX_MAT_SINGLE_LAYER:
     case RPX_MAT_COATED_DISPERSIVE: {
-        if constexpr ((F & M_COATED) == 0) return;
-        const double wavelength = wavelengths[in.wl_idx];
-        Sides sd = material_indices(m, wavelength);
-        V3 in_dir = norm(v3_of(in.direction));
+        if constexpr ((F & (M_FRESNEL | M_COATED)) == 0) return;
+        const bool film = m.type == RPX_MAT_SINGLE_LAYER || m.type == RPX_MAT_COATED_DISPERSIVE;
+        const double wavelength = m.type == RPX_MAT_FULL_DIELECTRIC ? 0.0 : wavelengths[in.wl_idx];
+        const Sides sd = material_indices(m, wavelength);
+        V3 in_dir = unit(v3_of(in.direction));
         RayS sp = begin_child(in, length, normal_f, point, idx);
         const Cf E1 = sp.E1, E2 = sp.E2;
         const double cosTheta = dot(normal, in_dir);
         const double cos1d = fabs(cosTheta);
-        const float cos1 = (float)cos1d;
-        const float sin1 = sqrtf((float)fabs(1 - cos1d * cos1d));
-        Cx n1d, n3d;
-        int flip;
-        if (cosTheta < 0.0) { n1d = sd.n_out; n3d = sd.n_in; flip = 1; }
-        else { n1d = sd.n_in; n3d = sd.n_out; flip = -1; }
-        const Cf n1 = cf_of(n1d), n2 = cf_of(sd.n_coat), n3 = cf_of(n3d);
-        const Cf n1s1 = cfscale(n1, sin1);
-        const Cf sin2 = cfdiv(n1s1, n2);
-        const Cf cos2 = cfsqrt(cfsub(cf(1, 0), cfmul(sin2, sin2)));
-        const Cf sin3 = cfdiv(n1s1, n3);
-        const Cf cos3 = cfsqrt(cfsub(cf(1, 0), cfmul(sin3, sin3)));
+        const bool inward = cosTheta < 0.0;
+        const Cx n1d = inward ? sd.n_out : sd.n_in, n3d = inward ? sd.n_in : sd.n_out;
+        const Cf n1 = cf_of(n1d), n3 = cf_of(n3d);
         const float P_in = n1.re * (cfabs2(E1) + cfabs2(E2));
         if (P_in == 0.0f) return;
-        const Cf n1cos1 = cfscale(n1, cos1), n2cos2 = cfmul(n2, cos2), n3cos3 = cfmul(n3, cos3);
-        const float dwc = (float)(2 * M_PI * m.thickness / wavelength);
-        const Cf phi = cfdiv(cfmul(cf(0.0f, -dwc), cfsub(n2, cfmul(sin2, sin2))), cos2);
-        const Cf ep1 = cfdiv(cfexp(phi), cfmul(cfscale(n2cos2, 4.0f), n3cos3));
-        const Cf ep2 = cfexp(cfscale(phi, -2.0f));
-        const Cf mep1 = cfneg(ep1);
-        // s-polarisation
-        Cf a = cfsub(n1cos1, n2cos2), b = cfadd(n1cos1, n2cos2);
-        Cf c = cfadd(n2cos2, n3cos3), d = cfsub(n2cos2, n3cos3);
-        Cf M00 = cfmul(mep1, cfadd(cfmul(a, c), cfmul(cfmul(b, d), ep2)));
-        Cf M01 = cfmul(ep1, cfadd(cfmul(cfmul(a, d), ep2), cfmul(b, c)));
-        Cf M10 = cfmul(ep1, cfadd(cfmul(a, d), cfmul(cfmul(b, c), ep2)));
-        Cf M11 = cfmul(mep1, cfadd(cfmul(cfmul(a, c), ep2), cfmul(b, d)));
-        Cf R_s = cfdiv(cfneg(M00), M01);
-        Cf T_s = cfadd(M10, cfmul(M11, R_s));
-        // p-polarisation
-        const Cf n1cos2 = cfmul(n1, cos2), n2cos1 = cfscale(n2, cos1);
-        const Cf n2cos3 = cfmul(n2, cos3), n3cos2 = cfmul(n3, cos2);
-        a = cfsub(n1cos2, n2cos1); b = cfadd(n1cos2, n2cos1);
-        c = cfadd(n2cos3, n3cos2); d = cfsub(n2cos3, n3cos2);
-        M00 = cfmul(mep1, cfadd(cfmul(a, c), cfmul(cfmul(b, d), ep2)));
-        M01 = cfmul(ep1, cfadd(cfmul(cfmul(a, d), ep2), cfmul(b, c)));
-        M10 = cfmul(ep1, cfadd(cfmul(a, d), cfmul(cfmul(b, c), ep2)));
-        M11 = cfmul(mep1, cfadd(cfmul(cfmul(a, c), ep2), cfmul(b, d)));
-        Cf R_p = cfdiv(cfneg(M00), M01);
-        Cf T_p = cfadd(M10, cfmul(M11, R_p));
-        R_s = cfmul(R_s, E1);
-        R_p = cfmul(R_p, E2);
-        if (power_frac_s(n1.re, R_s, R_p, P_in) > (float)m.reflection_threshold) {
-            RayS cr = sp;
-            cr.direction = f3_of(reflect_dir(in_dir, normal, cosTheta));
-            cr.E1 = R_s;
-            cr.E2 = cfneg(R_p);
-            cr.n = n1;
-            cr.ray_type_id |= RPX_REFL_RAY;
-            emit(cr);
-            sp = cr;
+        const float per_P = 1.0f / P_in;
+        const V3 tangent = sub(in_dir, mul(normal, cosTheta));
+        const V3 tg2 = mul(tangent, n1d.re / n3d.re);
+        const double tan_mag_sq = mag_sq(tg2);
+        const double c2 = sqrt(1 - tan_mag_sq);
+        const float cos1 = (float)cos1d, sin1 = sqrtf((float)fabs(1 - cos1d * cos1d));
+        bool real = n1.im == 0.0f && n3.im == 0.0f && n1.re > 0.0f && n3.re > 0.0f && tan_mag_sq < 1.0;
+        CoefsS k;
+        if (film) {
+            if constexpr ((F & M_COATED) != 0) {
+                const Cf n2 = cf_of(sd.n_coat);
+                const double sin1sq = mag_sq(tangent);
+                real = real && n2.im == 0.0f && n2.re > 0.0f &&
+                       n1d.re * n1d.re * sin1sq < sd.n_coat.re * sd.n_coat.re;
+                k = film_coefs_s(n1, n2, n3, cos1, sin1, (float)(2 * M_PI * m.thickness / wavelength), real,
+                                 (float)sin1sq, (float)c2);
+            } else {
+                return;
+            }
+        } else {
+            if constexpr ((F & M_FRESNEL) != 0)
+                k = fresnel_coefs_s(n1, n3, cos1, sin1, real, (float)c2);
+            else
+                return;
         }
-        const V3 t = refract_dir(in_dir, normal, cosTheta, n1d.re / n3d.re, flip);
-        const float aspect = sqrtf(cos3.re / cos1);
-        T_s = cfmul(T_s, cfscale(E1, aspect));
-        T_p = cfmul(T_p, cfscale(E2, aspect));
-        if (power_frac_s(n3.re, T_s, T_p, P_in) > (float)m.transmission_threshold) {
-            sp.direction = f3_of(t);
+        const Cf R_s = cfmul(k.rs, E1), R_p = cfmul(k.rp, E2);
+        if (n1.re * (cfabs2(R_s) + cfabs2(R_p)) * per_P > (float)m.reflection_threshold) {
+            sp.direction = f3_of(reflect_dir(in_dir, normal, cosTheta));
+            sp.E1 = R_s;
+            sp.E2 = cfneg(R_p);
+            sp.n = n1;
+            sp.ray_type_id |= RPX_REFL_RAY;
+            emit(sp);
+        }
+        const Cf T_s = cfmul(k.ts, E1), T_p = cfmul(k.tp, E2);
+        if (n3.re * (cfabs2(T_s) + cfabs2(T_p)) * per_P > (float)m.transmission_threshold) {
+            sp.direction = f3_of(sub(tg2, mul(normal, inward ? c2 : -c2)));
             sp.E1 = T_s;
             sp.E2 = T_p;
             sp.n = n3;

@@ -46,17 +46,36 @@ RPX_DEV rpx_rays_split_t advance_split(rpx_rays_split_t r, uint64_t off) {
 
 // Collects the (at most two) children of one ray as a two-slot shift
 // register (r0 latest), which the compiler keeps in registers.
-struct PairEmitS {
+struct PairEmitS {   // as PairEmit (rpx_materials.h): shared fields once, two slots
     static constexpr int kCap = 2;
-    RayS r0, r1;
+    struct Slot {
+        F3 direction;
+        Cf n, E1, E2;
+        double phase;
+        uint32_t type;
+    };
+    RayS shared;
+    Slot s0, s1;
     int n = 0;
     RPX_DEV void operator()(const RayS &x) {
-        r1 = r0;
-        r0 = x;
+        shared = x;
+        s1 = s0;
+        s0 = Slot{x.direction, x.n, x.E1, x.E2, x.phase, x.ray_type_id};
         ++n;
     }
     RPX_DEV void skip() { ++n; }
-    RPX_DEV const RayS &first() const { return n > 1 ? r1 : r0; }
+    RPX_DEV RayS child(const Slot &s) const {
+        RayS r = shared;
+        r.direction = s.direction;
+        r.n = s.n;
+        r.E1 = s.E1;
+        r.E2 = s.E2;
+        r.phase = s.phase;
+        r.ray_type_id = s.type;
+        return r;
+    }
+    RPX_DEV RayS first() const { return child(n > 1 ? s1 : s0); }
+    RPX_DEV RayS second() const { return child(s0); }
 };
 
 // After a generation's children are placed: stores children from index 2 on
@@ -76,8 +95,8 @@ struct TailEmitS {
 // Rays per tile (= workgroup size) of each split variant.  The lens
 // variants run 4 waves per SIMD, which two 512-lane workgroups fill exactly;
 // their tiles of 512 rays halve the per-tile look-back and staging work and
-// measured 4 % faster on C2 than tiles of 256.  V_FLAT (3 waves per SIMD)
-// and V_ALL (2) keep 256, which their occupancy divides.
+// measured 4 % faster on C2 than tiles of 256.  V_FLAT and V_ALL
+// (3 waves per SIMD) keep 256, which their occupancy divides.
 template <uint32_t F>
 constexpr int split_block() {
     return (F == V_SPHERES || F == V_LENS) ? 512 : RPX_BLOCK;
@@ -87,7 +106,7 @@ static uint32_t split_block_of(uint32_t variant) {
 }
 
 template <uint32_t F>
-__global__ __launch_bounds__(split_block<F>()) __attribute__((amdgpu_waves_per_eu(F == V_ALL ? 1 : F == V_FLAT ? 3 : 4)))
+__global__ __launch_bounds__(split_block<F>()) __attribute__((amdgpu_waves_per_eu(F == V_ALL || F == V_FLAT ? 3 : 4)))
 void k_generation_split(SplitArgs A) {
     constexpr int B = split_block<F>();
     __shared__ SceneLds lds_scene;
@@ -149,38 +168,16 @@ void k_generation_split(SplitArgs A) {
         }
         const V3 origin = v3_of(o32);
         const V3 dir = v3_of(d32);
-        double length = A.max_length;
-        uint32_t end_face = RPX_NO_FACE;
-        const V3 point = add(origin, mul(dir, A.max_length));
-        const int l0 = A.one_list < 0 ? 0 : A.one_list;
-        const int l1 = A.one_list < 0 ? S.n_face_lists : A.one_list + 1;
-        for (int l = l0; l < l1; ++l) {
-            const rpx_face_list_t &fl = S.face_lists[l];
-            const V3 p1 = transform(fl.inv_trans, origin);
-            const V3 p2 = transform(fl.inv_trans, point);
-            const double slen = sep(p1, p2), zrate = (p2.z - p1.z) / slen;
-            const int k0 = A.one_list < 0 ? fl.first_face : fl.first_face + A.one_face;
-            const int k1 = A.one_list < 0 ? fl.first_face + fl.n_faces : k0 + 1;
-            for (int k = k0; k < k1; ++k) {
-                auto test = [&](const rpx_face_t &fc) {
-                    if (face_out_of_reach(fc, p1.z, zrate * length, slen)) return;
-                    const double dist = face_intersect<F>(S, fc, p1, p2, 1);
-                    if (fc.tolerance < dist && dist < length) {
-                        length = dist;
-                        end_face = (uint32_t)fc.global_idx;
-                        hit_rec = k;
-                        hit_list = l;
-                    }
-                };
-                // k is the same in every lane: the lens and sphere variants
-                // read the face record with scalar loads (SGPRs, not VGPRs,
-                // hold its parameters through the root solve), which lets
-                // them run 4 waves per SIMD; the all-features variant reads
-                // the LDS copy
-                if constexpr (F == V_ALL) test(S.faces[k]);
-                else test(face_uniform(A.S.faces, k));
-            }
-        }
+        // the lens and sphere variants read the face records with scalar
+        // loads (SGPRs, not VGPRs, hold the parameters through the root
+        // solve), which lets them run 4 waves per SIMD; the all-features
+        // variant reads the LDS copy
+        const NearHit nh = nearest_face<F, F != V_ALL>(S, A.S.faces, origin, dir, A.max_length, A.max_length,
+                                                       A.one_list, A.one_face);
+        const double length = nh.length;
+        const uint32_t end_face = nh.end_face;
+        hit_rec = nh.rec;
+        hit_list = nh.list;
         in.f32[RPX_S_LENGTH * c + i] = (float)length;
         in.u32[RPX_END_FACE_IDX * c + i] = end_face;
         hit_length = length;
@@ -215,7 +212,7 @@ void k_generation_split(SplitArgs A) {
     __syncthreads();
     const uint64_t pos = lds_excl + local;
     if (count > 0 && pos < out_limit) store_ray_s(out, pos, ce.first());
-    if (count > 1 && pos + 1 < out_limit) store_ray_s(out, pos + 1, ce.r0);
+    if (count > 1 && pos + 1 < out_limit) store_ray_s(out, pos + 1, ce.second());
     if constexpr ((F & M_GRATING) != 0) {
         if (count > 2 && pos + 2 < out_limit) {
             // the third child is built again now that its position is known

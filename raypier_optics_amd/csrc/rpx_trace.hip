@@ -276,7 +276,19 @@ extern "C" rpx_status_t rpx_scene_create(const rpx_scene_desc_t *d, rpx_scene_t 
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1)
         return set_error(RPX_E_NO_DEVICE, "no HIP device");
     std::vector<char> blob;
-    size_t o_fl = push_table(blob, d->face_lists, d->n_face_lists);
+    // frames that are the global one are marked: the kernels use points and
+    // directions in them as they are
+    std::vector<rpx_face_list_t> lists(d->face_lists, d->face_lists + d->n_face_lists);
+    auto identity = [](const rpx_transform_t &t) {
+        for (int k = 0; k < 9; ++k)
+            if (t.m[k] != (k % 4 == 0 ? 1.0 : 0.0)) return false;
+        return t.t[0] == 0.0 && t.t[1] == 0.0 && t.t[2] == 0.0;
+    };
+    for (rpx_face_list_t &fl : lists) {
+        fl.pad[0] = (identity(fl.inv_trans) ? FL_INV_IDENTITY : 0) | (identity(fl.trans) ? FL_TRANS_IDENTITY : 0);
+        fl.pad[1] = 0;
+    }
+    size_t o_fl = push_table(blob, lists.data(), d->n_face_lists);
     size_t o_f = push_table(blob, d->faces, d->n_faces);
     size_t o_m = push_table(blob, d->materials, d->n_materials);
     size_t o_s = push_table(blob, d->shape_ops, d->n_shape_ops);
@@ -502,43 +514,13 @@ __global__ __launch_bounds__(RPX_BLOCK) void k_gausslet_generation(TraceArgs A) 
         // the input, children are written so), which keeps a generation
         // repeatable after a run-out look-back (its in-place lengths are then
         // not read back)
-        double length = A.link ? A.max_length : f[RPX_LENGTH * c + i];
-        uint32_t end_face = RPX_NO_FACE;
-        V3 point = add(origin, mul(dir, A.max_length));
-        if (A.one_list < 0) {
-            // trace_segment_c / FaceList.intersect_c (ctracer.pyx:2093-2104, 1882-1904)
-            for (int l = 0; l < S.n_face_lists; ++l) {
-                const rpx_face_list_t &fl = S.face_lists[l];
-                V3 p1 = transform(fl.inv_trans, origin);
-                V3 p2 = transform(fl.inv_trans, point);
-                const double slen = sep(p1, p2), zrate = (p2.z - p1.z) / slen;
-                for (int k = fl.first_face; k < fl.first_face + fl.n_faces; ++k) {
-                    const rpx_face_t &fc = S.faces[k];
-                    if (face_out_of_reach(fc, p1.z, zrate * length, slen)) continue;
-                    double dist = face_intersect<F>(S, fc, p1, p2, 1);
-                    if (fc.tolerance < dist && dist < length) {
-                        length = dist;
-                        end_face = (uint32_t)fc.global_idx;
-                        hit_rec = k;
-                        hit_list = l;
-                    }
-                }
-            }
-        } else {
-            // FaceList.intersect_one_face_c (ctracer.pyx:1861-1879)
-            const rpx_face_list_t &fl = S.face_lists[A.one_list];
-            const int k = fl.first_face + A.one_face;
-            const rpx_face_t &fc = S.faces[k];
-            V3 p1 = transform(fl.inv_trans, origin);
-            V3 p2 = transform(fl.inv_trans, point);
-            double dist = face_intersect<F>(S, fc, p1, p2, 1);
-            if (fc.tolerance < dist && dist < length) {
-                length = dist;
-                end_face = (uint32_t)fc.global_idx;
-                hit_rec = k;
-                hit_list = A.one_list;
-            }
-        }
+        const NearHit nh = nearest_face<F, F != V_ALL>(S, A.S.faces, origin, dir, A.max_length,
+                                                       A.link ? A.max_length : f[RPX_LENGTH * c + i], A.one_list,
+                                                       A.one_face);
+        const double length = nh.length;
+        const uint32_t end_face = nh.end_face;
+        hit_rec = nh.rec;
+        hit_list = nh.list;
         in.f64[RPX_LENGTH * c + i] = length;
         in.u32[RPX_END_FACE_IDX * c + i] = end_face;
         if (hit_rec >= 0) {
@@ -556,9 +538,7 @@ __global__ __launch_bounds__(RPX_BLOCK) void k_gausslet_generation(TraceArgs A) 
                 V3 pd = v3(P[(b + 3) * c + i], P[(b + 4) * c + i], P[(b + 5) * c + i]);
                 double plen = A.link ? A.max_length : P[(b + 9) * c + i];
                 V3 pend = add(po, mul(pd, A.max_length));
-                V3 q1 = transform(fl.inv_trans, po);
-                V3 q2 = transform(fl.inv_trans, pend);
-                double dist = face_intersect<F>(S, fc, q1, q2, 0);
+                double dist = face_intersect<F>(S, fc, make_seg(to_local(fl, po), to_local(fl, pend)), 0);
                 if (fc.tolerance < dist && dist < plen) {
                     in.para[(b + 9) * c + i] = dist;
                 } else {
@@ -653,8 +633,17 @@ __global__ __launch_bounds__(RPX_BLOCK) void k_gausslet_generation(TraceArgs A) 
     }
 }
 
+// Bound by latency: a wave spends over half its life waiting for its rays, the
+// scene and the look-back, so what it costs is its life times the waves a SIMD
+// holds.  Four waves (three for V_ALL) fit since the children take 66
+// registers and the common interfaces are evaluated in real numbers (168 and
+// 256 registers before, 126 and 168 now, with a few spills on the complex and
+// library paths), and a lens generation issues 1,400-1,775 vector instructions
+// per wave where it issued 2,330.  MI355X, 4,194,304 rays of the asphere and
+// doublet: 0.61-0.66 -> 0.50-0.55 ms per generation; Michelson, 65,536 rays to
+// depth 12: 16.0 -> 12.2 ms per trace.
 template <uint32_t F>
-__global__ __launch_bounds__(RPX_BLOCK) __attribute__((amdgpu_waves_per_eu(F == V_ALL ? 1 : 3)))
+__global__ __launch_bounds__(RPX_BLOCK) __attribute__((amdgpu_waves_per_eu(F == V_ALL ? 3 : 4)))
 void k_generation(TraceArgs A) {
     __shared__ SceneLds lds_scene;
     __shared__ uint32_t lds_hist[RPX_LDS_FACES];
@@ -716,43 +705,12 @@ void k_generation(TraceArgs A) {
             origin = v3(f[RPX_OX * c + i], f[RPX_OY * c + i], f[RPX_OZ * c + i]);
             dir = v3(f[RPX_DX * c + i], f[RPX_DY * c + i], f[RPX_DZ * c + i]);
         }
-        double length = A.max_length;
-        uint32_t end_face = RPX_NO_FACE;
-        V3 point = add(origin, mul(dir, A.max_length));
-        if (A.one_list < 0) {
-            // trace_segment_c / FaceList.intersect_c (ctracer.pyx:2093-2104, 1882-1904)
-            for (int l = 0; l < S.n_face_lists; ++l) {
-                const rpx_face_list_t &fl = S.face_lists[l];
-                V3 p1 = transform(fl.inv_trans, origin);
-                V3 p2 = transform(fl.inv_trans, point);
-                const double slen = sep(p1, p2), zrate = (p2.z - p1.z) / slen;
-                for (int k = fl.first_face; k < fl.first_face + fl.n_faces; ++k) {
-                    const rpx_face_t &fc = S.faces[k];
-                    if (face_out_of_reach(fc, p1.z, zrate * length, slen)) continue;
-                    double dist = face_intersect<F>(S, fc, p1, p2, 1);
-                    if (fc.tolerance < dist && dist < length) {
-                        length = dist;
-                        end_face = (uint32_t)fc.global_idx;
-                        hit_rec = k;
-                        hit_list = l;
-                    }
-                }
-            }
-        } else {
-            // FaceList.intersect_one_face_c (ctracer.pyx:1861-1879)
-            const rpx_face_list_t &fl = S.face_lists[A.one_list];
-            const int k = fl.first_face + A.one_face;
-            const rpx_face_t &fc = S.faces[k];
-            V3 p1 = transform(fl.inv_trans, origin);
-            V3 p2 = transform(fl.inv_trans, point);
-            double dist = face_intersect<F>(S, fc, p1, p2, 1);
-            if (fc.tolerance < dist && dist < length) {
-                length = dist;
-                end_face = (uint32_t)fc.global_idx;
-                hit_rec = k;
-                hit_list = A.one_list;
-            }
-        }
+        const NearHit nh = nearest_face<F, F != V_ALL>(S, A.S.faces, origin, dir, A.max_length, A.max_length,
+                                                       A.one_list, A.one_face);
+        const double length = nh.length;
+        const uint32_t end_face = nh.end_face;
+        hit_rec = nh.rec;
+        hit_list = nh.list;
         in.f64[RPX_LENGTH * c + i] = length;
         in.u32[RPX_END_FACE_IDX * c + i] = end_face;
         if (hit_rec >= 0) {
@@ -786,7 +744,7 @@ void k_generation(TraceArgs A) {
     __syncthreads();
     const uint64_t pos = lds_excl + local;
     if (count > 0 && pos < out_limit) store_ray(out, pos, ce.first());
-    if (count > 1 && pos + 1 < out_limit) store_ray(out, pos + 1, ce.r0);
+    if (count > 1 && pos + 1 < out_limit) store_ray(out, pos + 1, ce.second());
     if constexpr ((F & M_GRATING) != 0) {
         if (count > 2 && pos + 2 < out_limit) {
             // the third child is built again now that its position is known
