@@ -350,12 +350,36 @@ rpx_status_t rpx_trace_rays(const rpx_scene_t *scene,
                             void *workspace, uint64_t workspace_bytes,
                             void *stream);
 
+/* rpx_trace_rays for a caller that has no use for the last generation's
+ * children: when max_generations generations are traced, those of the last one
+ * are neither stored nor evaluated, and counts[max_generations] is 0. */
+rpx_status_t rpx_trace_rays_discard(const rpx_scene_t *scene,
+                            const rpx_rays_t *in, uint64_t n_in,
+                            float max_length,
+                            const double *wavelengths, uint64_t n_wavelengths,
+                            int32_t max_generations, rpx_rays_t *pool,
+                            uint64_t *counts, uint64_t *offsets, int32_t *n_traced,
+                            uint32_t *face_hits,
+                            void *workspace, uint64_t workspace_bytes,
+                            void *stream);
+
 /* The same loop for a gausslet collection (core/tracer.py:9-47 with
  * ctracer.pyx:2214-2282 per generation: trace_gausslet_c and the parabasal
  * rays), as rpx_trace_rays with gausslet buffers (`para` set on `in` and the
  * pool) and max_length in double precision (as rpx_trace_gausslet).  For scenes without a decomposition (ResampleGaussletMaterial)
  * face, whose captures need the host between generations. */
 rpx_status_t rpx_trace_gausslets(const rpx_scene_t *scene,
+                            const rpx_rays_t *in, uint64_t n_in,
+                            double max_length,
+                            const double *wavelengths, uint64_t n_wavelengths,
+                            int32_t max_generations, rpx_rays_t *pool,
+                            uint64_t *counts, uint64_t *offsets, int32_t *n_traced,
+                            uint32_t *face_hits,
+                            void *workspace, uint64_t workspace_bytes,
+                            void *stream);
+
+/* As rpx_trace_rays_discard. */
+rpx_status_t rpx_trace_gausslets_discard(const rpx_scene_t *scene,
                             const rpx_rays_t *in, uint64_t n_in,
                             double max_length,
                             const double *wavelengths, uint64_t n_wavelengths,
@@ -622,6 +646,17 @@ rpx_status_t rpx_trace_segment_split(const rpx_scene_t *scene,
  * workspace rpx_chain_workspace_bytes(max(n_in, pool->capacity),
  * max_generations) bytes).  No counterpart in the reference. */
 rpx_status_t rpx_trace_rays_split(const rpx_scene_t *scene,
+                                  const rpx_rays_split_t *in, uint64_t n_in,
+                                  float max_length,
+                                  const double *wavelengths, uint64_t n_wavelengths,
+                                  int32_t max_generations, rpx_rays_split_t *pool,
+                                  uint64_t *counts, uint64_t *offsets, int32_t *n_traced,
+                                  uint32_t *face_hits,
+                                  void *workspace, uint64_t workspace_bytes,
+                                  void *stream);
+
+/* As rpx_trace_rays_discard. */
+rpx_status_t rpx_trace_rays_split_discard(const rpx_scene_t *scene,
                                   const rpx_rays_split_t *in, uint64_t n_in,
                                   float max_length,
                                   const double *wavelengths, uint64_t n_wavelengths,

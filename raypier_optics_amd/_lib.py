@@ -112,6 +112,9 @@ _SIGNATURES = {
     "rpx_sum_gaussian_modes_noalloc": (c_i32, [P(_abi.Rays), c_u64, c_void_p, c_void_p, c_u64, c_void_p, c_u64,
                                                c_f64, c_void_p, c_i32, c_void_p]),
 }
+# the loops for callers that discard the last generation's children
+for _name in ("rpx_trace_rays", "rpx_trace_gausslets", "rpx_trace_rays_split"):
+    _SIGNATURES[_name + "_discard"] = _SIGNATURES[_name]
 
 EXPORTED = sorted(_SIGNATURES)
 

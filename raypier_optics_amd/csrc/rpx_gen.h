@@ -85,42 +85,36 @@ static Workspace carve(void *ws, uint64_t n_in) {
     return w;
 }
 
-// Stage face lists and faces in LDS; hand back a view that points there.
-// LDS copy of a scene's small tables.  Faces and face lists always fit
-// (validated at scene creation); materials and shape programs are staged when
-// they fit and otherwise read from global memory.
-#define RPX_LDS_MATERIALS 8
-#define RPX_LDS_SHAPE_OPS 32
+// LDS copy of a scene's small tables.  Face lists and faces always fit
+// (validated at scene creation); shape programs and materials are staged when
+// they fit too (scene creation decides) and otherwise read from global memory.
+// The staged tables are one block in device memory, copied in 16-byte units
+// with all of a lane's loads in flight together: copying table by table cost a
+// memory round trip each, five per workgroup.
+#define RPX_LDS_SCENE 21248
 struct SceneLds {
-    rpx_face_t faces[RPX_LDS_FACES];
-    rpx_face_list_t lists[RPX_LDS_LISTS];
-    rpx_material_t materials[RPX_LDS_MATERIALS];
-    rpx_shape_op_t shape_ops[RPX_LDS_SHAPE_OPS];
+    uint4 block[RPX_LDS_SCENE / 16];
 };
 
-template <class T>
-static __device__ __forceinline__ void lds_copy(T *dst, const T *src, int n) {
-    static_assert(sizeof(T) % 8 == 0, "tables are copied as doubles");
-    const int nw = n * (int)(sizeof(T) / 8);
-    const double *s = (const double *)src;
-    double *d = (double *)dst;
-    for (int k = threadIdx.x; k < nw; k += blockDim.x) d[k] = s[k];
-}
-
-// Stage the scene in LDS; hand back a view that points there.  Ends with a
-// workgroup barrier.
+// Copies the scene's block to LDS; hands back a view that points there.  The
+// caller's next workgroup barrier completes the copy.
 static __device__ __forceinline__ SceneView stage_scene(const SceneView &S, SceneLds &L) {
-    lds_copy(L.faces, S.faces, S.n_faces);
-    lds_copy(L.lists, S.face_lists, S.n_face_lists);
-    const bool mats = S.n_materials <= RPX_LDS_MATERIALS, ops = S.n_shape_ops <= RPX_LDS_SHAPE_OPS;
-    if (mats) lds_copy(L.materials, S.materials, S.n_materials);
-    if (ops) lds_copy(L.shape_ops, S.shape_ops, S.n_shape_ops);
-    __syncthreads();
+    const uint4 *src = (const uint4 *)S.face_lists;
+    const int n = S.stage_units, step = blockDim.x, k = threadIdx.x;
+    uint4 a, b, c;
+    if (k < n) a = src[k];
+    if (k + step < n) b = src[k + step];
+    if (k + 2 * step < n) c = src[k + 2 * step];
+    if (k < n) L.block[k] = a;
+    if (k + step < n) L.block[k + step] = b;
+    if (k + 2 * step < n) L.block[k + 2 * step] = c;
+    for (int q = k + 3 * step; q < n; q += step) L.block[q] = src[q];
     SceneView v = S;
-    v.faces = L.faces;
-    v.face_lists = L.lists;
-    if (mats) v.materials = L.materials;
-    if (ops) v.shape_ops = L.shape_ops;
+    const char *base = (const char *)L.block;
+    v.face_lists = (const rpx_face_list_t *)base;
+    v.faces = (const rpx_face_t *)(base + S.n_face_lists * sizeof(rpx_face_list_t));
+    if (S.stage_materials >= 0) v.materials = (const rpx_material_t *)(base + S.stage_materials);
+    if (S.stage_ops >= 0) v.shape_ops = (const rpx_shape_op_t *)(base + S.stage_ops);
     return v;
 }
 
@@ -463,7 +457,7 @@ struct ChainGen {
     uint64_t *tile_status;
     uint64_t tag;
     GenControl *head_out;
-    int32_t in_pool, store_children;
+    int32_t in_pool, store_children, count_children;
     uint32_t tile_base;
     int32_t by_launch;
     uint64_t lookback_ticks;
@@ -490,6 +484,7 @@ struct ChainSpec {
     uint64_t n_in, pool_rays, max_children;
     uint32_t block = RPX_BLOCK;               // rays per tile of the generation kernel (<= the workspace's)
     bool bytes_per_parent = false;            // bytes_hit per gausslet with children (gausslet chains)
+    bool count_last = true;                   // evaluate and count the last generation's children
     int32_t max_generations;
     int timing_slot;                          // RPX_TIMING_* of the generation kernel
     double bytes_in, bytes_hit, bytes_child;  // algorithmic bytes per input ray / hit / child
@@ -594,6 +589,7 @@ static rpx_status_t run_chain_once(const ChainSpec &c, const rpx_scene_t *scene,
         cg.head_out = heads_dev + g;
         cg.in_pool = g > 0;
         cg.store_children = g + 1 < L ? 1 : 0;
+        cg.count_children = (g + 1 < L || c.count_last) ? 1 : 0;
         cg.tile_base = 0;
         cg.by_launch = by_launch ? 1 : 0;
         cg.lookback_ticks = by_launch ? ticks : 0;
@@ -711,6 +707,7 @@ static rpx_status_t run_chain_once(const ChainSpec &c, const rpx_scene_t *scene,
             for (int s2 = 0; s2 < RPX_SHARDS; ++s2) hits += heads[g].hit_shards[s2];
             if (c.bytes_per_parent) hits = heads[g].parents;
             const bool stored = g + 1 < L;
+            if (!stored && !c.count_last) hits = 0;
             rpx_timing_add(c.timing_slot, ms, (double)counts[g] * c.bytes_in + (double)hits * c.bytes_hit +
                                                   (stored ? (double)counts[g + 1] * c.bytes_child : 0.0));
         }

@@ -175,6 +175,10 @@ struct SceneView {
     int32_t n_face_lists, n_faces, n_materials, n_shape_ops, n_vertices;
     int32_t n_zernikes;
     int32_t n_list_faces;   // faces that belong to face lists (chain order)
+    // the tables a workgroup stages in LDS: the first stage_units 16-byte units
+    // of the block that starts with the face lists, then the faces; shape_ops
+    // and materials are at these byte offsets in it, or not staged (-1)
+    int32_t stage_units, stage_ops, stage_materials;
     int32_t max_children;
 };
 

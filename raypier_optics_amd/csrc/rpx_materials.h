@@ -108,6 +108,25 @@ RPX_DEV Ray load_ray(const rpx_rays_t &r, uint64_t i) {
     return o;
 }
 
+// The fields of ray i that its children depend on besides its geometry and
+// wavelength index; the others are left unset.
+RPX_DEV Ray load_ray_rest(const rpx_rays_t &r, uint64_t i) {
+    const double *f = r.f64;
+    const uint64_t c = r.capacity;
+    Ray o;
+    o.normal = v3(0, 0, 0);
+    o.E_vector = v3(f[RPX_EX * c + i], f[RPX_EY * c + i], f[RPX_EZ * c + i]);
+    o.n = cx(f[RPX_N_RE * c + i], f[RPX_N_IM * c + i]);
+    o.E1 = cx(f[RPX_E1_RE * c + i], f[RPX_E1_IM * c + i]);
+    o.E2 = cx(f[RPX_E2_RE * c + i], f[RPX_E2_IM * c + i]);
+    o.phase = f[RPX_PHASE * c + i];
+    o.accum = f[RPX_ACCUM * c + i];
+    o.parent_idx = 0;
+    o.ray_ident = r.u32[RPX_RAY_IDENT * c + i];
+    o.ray_type_id = r.u32[RPX_RAY_TYPE_ID * c + i];
+    return o;
+}
+
 RPX_DEV void store_ray(const rpx_rays_t &r, uint64_t i, const Ray &o) {
     double *f = r.f64;
     const uint64_t c = r.capacity;
@@ -220,6 +239,12 @@ struct WlTable {
     RPX_DEV double operator[](uint32_t i) const { return (i < n) ? wl[i] : __builtin_nan(""); }
 };
 
+// The wavelength of one ray, looked up beforehand.
+struct WlOne {
+    double v;
+    RPX_DEV double operator[](uint32_t) const { return v; }
+};
+
 // Whether a material can have children: OpaqueMaterial and the base
 // InterfaceMaterial never do, so a ray ending on them needs no material
 // evaluation and none of its record beyond the geometry.
@@ -322,9 +347,9 @@ RPX_DEV Coefs film_coefs(Cx n1, Cx n2, Cx n3, double cos1, double sin1, double d
 // DiffractionGratingMaterial.eval_child_ray_c (cmaterials.pyx:1472-1542):
 // one child per propagating order, orders in list order (one order in the
 // reference); children past the emitter's kCap are counted, not built.
-template <class Emit>
+template <class W, class Emit>
 RPX_DEV void grating_children(const rpx_material_t &m, const Ray &in, uint32_t idx, V3 point,
-                              const Orientation &orient, const WlTable &wavelengths, Emit &emit) {
+                              const Orientation &orient, const W &wavelengths, Emit &emit) {
     V3 normal = unit(orient.normal);
     V3 tangent = unit(orient.tangent);
     V3 tangent2 = cross(normal, tangent);
@@ -369,9 +394,9 @@ RPX_DEV void grating_children(const rpx_material_t &m, const Ray &in, uint32_t i
     }
 }
 
-template <uint32_t F, class Emit>
+template <uint32_t F, class W, class Emit>
 RPX_DEV void eval_children(const rpx_material_t &m, const Ray &in, uint32_t idx, V3 point,
-                           const Orientation &orient, const WlTable &wavelengths, Emit &emit) {
+                           const Orientation &orient, const W &wavelengths, Emit &emit) {
     switch (m.type) {
     case RPX_MAT_TRANSPARENT: {
         if constexpr ((F & M_SIMPLE) == 0) return;  // cmaterials.pyx:260-278

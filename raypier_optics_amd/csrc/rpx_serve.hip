@@ -193,7 +193,8 @@ void k_batch(const BatchJob *jobs, BatchControl *ctl, uint64_t *status,
         if (tile >= total) return;
         const int j = lds_job;
         const BatchJob &J = jobs[j];
-        const SceneView S = stage_scene(J.S, lds_scene);   // ends with a barrier
+        const SceneView S = stage_scene(J.S, lds_scene);
+        __syncthreads();
         const uint64_t i = (tile - J.tile_begin) * RPX_BLOCK + threadIdx.x;
         PairEmit ce;
         bool hit = false;

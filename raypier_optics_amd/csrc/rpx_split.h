@@ -102,6 +102,25 @@ RPX_DEV RayS load_ray_s(const rpx_rays_split_t &r, uint64_t i) {
     return o;
 }
 
+// The fields that children depend on besides geometry and wavelength index
+// (as load_ray_rest).
+RPX_DEV RayS load_ray_rest_s(const rpx_rays_split_t &r, uint64_t i) {
+    const float *f = r.f32;
+    const uint64_t c = r.capacity;
+    RayS o;
+    o.normal = f3(0, 0, 0);
+    o.E_vector = f3(f[RPX_S_EX * c + i], f[RPX_S_EY * c + i], f[RPX_S_EZ * c + i]);
+    o.n = cf(f[RPX_S_N_RE * c + i], f[RPX_S_N_IM * c + i]);
+    o.E1 = cf(f[RPX_S_E1_RE * c + i], f[RPX_S_E1_IM * c + i]);
+    o.E2 = cf(f[RPX_S_E2_RE * c + i], f[RPX_S_E2_IM * c + i]);
+    o.phase = r.f64[RPX_S_PHASE * c + i];
+    o.accum = r.f64[RPX_S_ACCUM * c + i];
+    o.parent_idx = 0;
+    o.ray_ident = r.u32[RPX_RAY_IDENT * c + i];
+    o.ray_type_id = r.u32[RPX_RAY_TYPE_ID * c + i];
+    return o;
+}
+
 RPX_DEV void store_ray_s(const rpx_rays_split_t &r, uint64_t i, const RayS &o) {
     float *f = r.f32;
     const uint64_t c = r.capacity;
@@ -247,9 +266,9 @@ RPX_DEV RayS begin_child(const RayS &in, double length, F3 normal_f, V3 point, u
 // The grating's children, FP32-split (the float64 grating_children's
 // emitter protocol: one child per propagating order, those past kCap
 // counted, not built).
-template <class Emit>
+template <class W, class Emit>
 RPX_DEV void grating_children_split(const rpx_material_t &m, const RayS &in, double length, uint32_t idx, V3 point,
-                                    const Orientation &orient, const WlTable &wavelengths, Emit &emit) {
+                                    const Orientation &orient, const W &wavelengths, Emit &emit) {
     const V3 normal = unit(orient.normal);
     const F3 normal_f = f3_of(normal);
     const V3 tangent = unit(orient.tangent);
@@ -289,9 +308,9 @@ RPX_DEV void grating_children_split(const rpx_material_t &m, const RayS &in, dou
 }
 
 // InterfaceMaterial.eval_child_ray_c of every material, FP32-split.
-template <uint32_t F, class Emit>
+template <uint32_t F, class W, class Emit>
 RPX_DEV void eval_children_split(const rpx_material_t &m, const RayS &in, double length, uint32_t idx,
-                                 V3 point, const Orientation &orient, const WlTable &wavelengths, Emit &emit) {
+                                 V3 point, const Orientation &orient, const W &wavelengths, Emit &emit) {
     const V3 normal = unit(orient.normal);
     const F3 normal_f = f3_of(normal);
     switch (m.type) {

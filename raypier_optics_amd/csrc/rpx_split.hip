@@ -28,6 +28,7 @@ struct SplitArgs {
     GenLink *link;
     uint64_t pool_rays;
     int32_t in_pool, store_children;
+    int32_t count_children = 1;   // as TraceArgs
     uint64_t status_tag;
     GenControl *head_out;
     // tile order, as TraceArgs
@@ -141,15 +142,18 @@ void k_generation_split(SplitArgs A) {
     const float *f = in.f32;
     const uint64_t c = in.capacity;
     F3 o32 = f3(0, 0, 0), d32 = f3(0, 0, 0);
+    uint32_t wl_idx = 0;
+    auto load_geometry = [&](uint64_t i) {
+        o32 = f3(f[RPX_S_OX * c + i], f[RPX_S_OY * c + i], f[RPX_S_OZ * c + i]);
+        d32 = f3(f[RPX_S_DX * c + i], f[RPX_S_DY * c + i], f[RPX_S_DZ * c + i]);
+        wl_idx = in.u32[RPX_WL_IDX * c + i];
+    };
     if (A.by_launch) {
         const uint64_t i0 = (uint64_t)my_tile * B + threadIdx.x;
-        if (i0 < n_in) {
-            o32 = f3(f[RPX_S_OX * c + i0], f[RPX_S_OY * c + i0], f[RPX_S_OZ * c + i0]);
-            d32 = f3(f[RPX_S_DX * c + i0], f[RPX_S_DY * c + i0], f[RPX_S_DZ * c + i0]);
-        }
+        if (i0 < n_in) load_geometry(i0);
     }
     const SceneView S = stage_scene(A.S, lds_scene);
-    for (int k = threadIdx.x; k < RPX_LDS_FACES; k += blockDim.x) lds_hist[k] = 0;
+    if (threadIdx.x < RPX_LDS_FACES) lds_hist[threadIdx.x] = 0;
     if (threadIdx.x == 0) {
         lds_tile = my_tile;
         lds_hits = 0;
@@ -161,11 +165,11 @@ void k_generation_split(SplitArgs A) {
     bool hit = false;
     int hit_rec = -1, hit_list = -1;
     double hit_length = 0;
+    const bool children = A.count_children;
     if (i < n_in) {
-        if (!A.by_launch) {
-            o32 = f3(f[RPX_S_OX * c + i], f[RPX_S_OY * c + i], f[RPX_S_OZ * c + i]);
-            d32 = f3(f[RPX_S_DX * c + i], f[RPX_S_DY * c + i], f[RPX_S_DZ * c + i]);
-        }
+        if (!A.by_launch) load_geometry(i);
+        // the wavelength arrives while the faces are searched
+        WlOne wavelength{children ? A.wavelengths[wl_idx] : 0.0};
         const V3 origin = v3_of(o32);
         const V3 dir = v3_of(d32);
         // the lens and sphere variants read the face records with scalar
@@ -184,62 +188,69 @@ void k_generation_split(SplitArgs A) {
         if (hit_rec >= 0) {
             atomicAdd(&lds_hist[hit_rec], 1u);
             const rpx_face_t &fc = S.faces[hit_rec];
-            if (fc.material >= 0 && material_emits(S.materials[fc.material])) {
+            if (children && fc.material >= 0 && material_emits(S.materials[fc.material])) {
                 hit = true;   // counted: the rest of its record is read
                 const rpx_face_list_t &fl = S.face_lists[hit_list];
-                RayS r = load_ray_s(in, i);
+                RayS r = load_ray_rest_s(in, i);
+                r.origin = o32;
+                r.direction = d32;
+                r.wl_idx = wl_idx;
                 r.length = (float)length;
                 r.end_face_idx = end_face;
                 const V3 hp = add(origin, mul(dir, length));
                 const Orientation o = compute_orientation<F>(S, fl, fc, hp);
-                eval_children_split<F>(S.materials[fc.material], r, length, (uint32_t)i, hp, o, A.wavelengths, ce);
+                eval_children_split<F>(S.materials[fc.material], r, length, (uint32_t)i, hp, o, wavelength, ce);
             }
         }
     }
-    // a multi-order grating (all-features variant only) can have a third child
-    const uint32_t count = (uint32_t)min(ce.n, (F & M_GRATING) ? 3 : 2);
-    uint32_t block_total;
-    const uint32_t local = block_scan_small(count, lds_wave, &block_total);
-    {
-        const uint64_t mh = __ballot(hit);
-        if ((threadIdx.x & 63) == 0) atomicAdd(&lds_hits, (uint32_t)__popcll(mh));
-    }
-    if (threadIdx.x < 64) {
-        const uint64_t excl = lookback_tagged(A.ws.tile_status, tile, 0, block_total, &A.ws.ctl->error, A.status_tag,
-                                              A.lookback_ticks);
-        if (threadIdx.x == 0) lds_excl = excl;
-    }
-    __syncthreads();
-    const uint64_t pos = lds_excl + local;
-    if (count > 0 && pos < out_limit) store_ray_s(out, pos, ce.first());
-    if (count > 1 && pos + 1 < out_limit) store_ray_s(out, pos + 1, ce.second());
-    if constexpr ((F & M_GRATING) != 0) {
-        if (count > 2 && pos + 2 < out_limit) {
-            // the third child is built again now that its position is known
-            const rpx_face_t &fc = S.faces[hit_rec];
-            RayS r = load_ray_s(in, i);
-            r.length = (float)hit_length;
-            const V3 hp = add(v3_of(r.origin), mul(v3_of(r.direction), hit_length));
-            const Orientation o = compute_orientation<F>(S, S.face_lists[hit_list], fc, hp);
-            TailEmitS te{&out, pos, out_limit};
-            grating_children_split(S.materials[fc.material], r, hit_length, (uint32_t)i, hp, o, A.wavelengths, te);
+    if (children) {
+        // a multi-order grating (all-features variant only) can have a third child
+        const uint32_t count = (uint32_t)min(ce.n, (F & M_GRATING) ? 3 : 2);
+        uint32_t block_total;
+        const uint32_t local = block_scan_small(count, lds_wave, &block_total);
+        {
+            const uint64_t mh = __ballot(hit);
+            if ((threadIdx.x & 63) == 0) atomicAdd(&lds_hits, (uint32_t)__popcll(mh));
         }
-    }
-    if (threadIdx.x == 0) {
-        // a chain's hit total is the sum of its face totals (k_chain_fold);
-        // one word per generation would take every tile's atomic in one line
-        if (!A.link) add_hits(A.ws.ctl, tile, lds_hits);
-        if ((uint64_t)tile == (n_in - 1) / B) {
-            const uint64_t kids = lds_excl + block_total;
-            A.ws.ctl->children = kids;
-            if (A.link) {
-                const uint64_t at = A.link[0].out_offset;
-                A.link[1].count = kids;
-                A.link[1].offset = at;
-                A.link[1].out_offset = at + kids;
-                A.head_out->children = kids;   // host-mapped: read once the generation has ended
+        if (threadIdx.x < 64) {
+            const uint64_t excl = lookback_tagged(A.ws.tile_status, tile, 0, block_total, &A.ws.ctl->error, A.status_tag,
+                                                  A.lookback_ticks);
+            if (threadIdx.x == 0) lds_excl = excl;
+        }
+        __syncthreads();
+        const uint64_t pos = lds_excl + local;
+        if (count > 0 && pos < out_limit) store_ray_s(out, pos, ce.first());
+        if (count > 1 && pos + 1 < out_limit) store_ray_s(out, pos + 1, ce.second());
+        if constexpr ((F & M_GRATING) != 0) {
+            if (count > 2 && pos + 2 < out_limit) {
+                // the third child is built again now that its position is known
+                const rpx_face_t &fc = S.faces[hit_rec];
+                RayS r = load_ray_s(in, i);
+                r.length = (float)hit_length;
+                const V3 hp = add(v3_of(r.origin), mul(v3_of(r.direction), hit_length));
+                const Orientation o = compute_orientation<F>(S, S.face_lists[hit_list], fc, hp);
+                TailEmitS te{&out, pos, out_limit};
+                grating_children_split(S.materials[fc.material], r, hit_length, (uint32_t)i, hp, o, A.wavelengths, te);
             }
         }
+        if (threadIdx.x == 0) {
+            // a chain's hit total is the sum of its face totals (k_chain_fold);
+            // one word per generation would take every tile's atomic in one line
+            if (!A.link) add_hits(A.ws.ctl, tile, lds_hits);
+            if ((uint64_t)tile == (n_in - 1) / B) {
+                const uint64_t kids = lds_excl + block_total;
+                A.ws.ctl->children = kids;
+                if (A.link) {
+                    const uint64_t at = A.link[0].out_offset;
+                    A.link[1].count = kids;
+                    A.link[1].offset = at;
+                    A.link[1].out_offset = at + kids;
+                    A.head_out->children = kids;   // host-mapped: read once the generation has ended
+                }
+            }
+        }
+    } else {
+        __syncthreads();   // lds_hist is complete
     }
     if (A.face_hits || A.link) {
         uint32_t *shard = A.ws.ctl->face_shards[tile % RPX_SHARDS];
@@ -408,11 +419,11 @@ extern "C" rpx_status_t rpx_trace_segment_split(const rpx_scene_t *scene, int32_
 
 // rpx_trace_rays_split: the FP32-split generations of trace_rays as one
 // device-resident chain (run_chain in rpx_gen.h).
-extern "C" rpx_status_t rpx_trace_rays_split(const rpx_scene_t *scene, const rpx_rays_split_t *in, uint64_t n_in,
-                                             float max_length, const double *wavelengths, uint64_t n_wavelengths,
-                                             int32_t max_generations, rpx_rays_split_t *pool, uint64_t *counts,
-                                             uint64_t *offsets, int32_t *n_traced, uint32_t *face_hits,
-                                             void *workspace, uint64_t workspace_bytes, void *stream_) {
+static rpx_status_t trace_rays_split_impl(const rpx_scene_t *scene, const rpx_rays_split_t *in, uint64_t n_in, float
+                                          max_length, const double *wavelengths, uint64_t n_wavelengths, int32_t
+                                          max_generations, rpx_rays_split_t *pool, uint64_t *counts, uint64_t
+                                          *offsets, int32_t *n_traced, uint32_t *face_hits, void *workspace, uint64_t
+                                          workspace_bytes, void *stream_, bool count_last) {
     if (!n_traced || !counts || !offsets)
         return rpx_set_error(RPX_E_INVALID, "counts / offsets / n_traced are null");
     *n_traced = 0;
@@ -435,6 +446,7 @@ extern "C" rpx_status_t rpx_trace_rays_split(const rpx_scene_t *scene, const rpx
     spec.bytes_in = 24.0 + 8.0;    // FP32-split geometry read, length + end face written
     spec.bytes_hit = 64.0;
     spec.bytes_child = 112.0;
+    spec.count_last = count_last;
     if (rpx_status_t st = check_chain(spec, scene, workspace, workspace_bytes)) return st;
     const uint32_t variant = split_variant(scene);
     spec.block = split_block_of(variant);
@@ -462,6 +474,7 @@ extern "C" rpx_status_t rpx_trace_rays_split(const rpx_scene_t *scene, const rpx
         A.in_pool = cg.in_pool;
         A.in = cg.in_pool ? *pool : *in;
         A.store_children = cg.store_children;
+        A.count_children = cg.count_children;
         A.tile_base = cg.tile_base;
         A.by_launch = cg.by_launch;
         A.lookback_ticks = cg.lookback_ticks;
@@ -470,3 +483,23 @@ extern "C" rpx_status_t rpx_trace_rays_split(const rpx_scene_t *scene, const rpx
     };
     return run_chain(spec, scene, workspace, launch, counts, offsets, n_traced, face_hits, (hipStream_t)stream_);
 }
+
+extern "C" rpx_status_t rpx_trace_rays_split(const rpx_scene_t *scene, const rpx_rays_split_t *in, uint64_t n_in,
+                                             float max_length, const double *wavelengths, uint64_t n_wavelengths,
+                                             int32_t max_generations, rpx_rays_split_t *pool, uint64_t *counts,
+                                             uint64_t *offsets, int32_t *n_traced, uint32_t *face_hits, void
+                                             *workspace, uint64_t workspace_bytes, void *stream_) {
+    return trace_rays_split_impl(scene, in, n_in, max_length, wavelengths, n_wavelengths, max_generations, pool,
+                                 counts, offsets, n_traced, face_hits, workspace, workspace_bytes, stream_, true);
+}
+
+extern "C" rpx_status_t rpx_trace_rays_split_discard(const rpx_scene_t *scene, const rpx_rays_split_t *in, uint64_t
+                                                     n_in, float max_length, const double *wavelengths, uint64_t
+                                                     n_wavelengths, int32_t max_generations, rpx_rays_split_t *pool,
+                                                     uint64_t *counts, uint64_t *offsets, int32_t *n_traced, uint32_t
+                                                     *face_hits, void *workspace, uint64_t workspace_bytes, void
+                                                     *stream_) {
+    return trace_rays_split_impl(scene, in, n_in, max_length, wavelengths, n_wavelengths, max_generations, pool,
+                                 counts, offsets, n_traced, face_hits, workspace, workspace_bytes, stream_, false);
+}
+

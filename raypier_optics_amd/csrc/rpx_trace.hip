@@ -288,10 +288,37 @@ extern "C" rpx_status_t rpx_scene_create(const rpx_scene_desc_t *d, rpx_scene_t 
         fl.pad[0] = (identity(fl.inv_trans) ? FL_INV_IDENTITY : 0) | (identity(fl.trans) ? FL_TRANS_IDENTITY : 0);
         fl.pad[1] = 0;
     }
-    size_t o_fl = push_table(blob, lists.data(), d->n_face_lists);
-    size_t o_f = push_table(blob, d->faces, d->n_faces);
-    size_t o_m = push_table(blob, d->materials, d->n_materials);
-    size_t o_s = push_table(blob, d->shape_ops, d->n_shape_ops);
+    // one block of face lists, faces and, as far as RPX_LDS_SCENE takes them,
+    // shape programs and materials (the other way round when the programs alone
+    // are long); each record is a multiple of 16 bytes
+    static_assert(sizeof(rpx_face_list_t) % 16 == 0 && sizeof(rpx_face_t) % 16 == 0 &&
+                  sizeof(rpx_shape_op_t) % 16 == 0 && sizeof(rpx_material_t) % 16 == 0, "staged in 16-byte units");
+    auto append = [&](const void *src, size_t bytes) {
+        const size_t off = blob.size();
+        blob.insert(blob.end(), (const char *)src, (const char *)src + bytes);
+        return off;
+    };
+    const size_t ops_bytes = sizeof(rpx_shape_op_t) * (size_t)d->n_shape_ops;
+    const size_t mat_bytes = sizeof(rpx_material_t) * (size_t)d->n_materials;
+    const size_t o_fl = append(lists.data(), sizeof(rpx_face_list_t) * lists.size());
+    const size_t o_f = append(d->faces, sizeof(rpx_face_t) * (size_t)d->n_faces);
+    const size_t fixed = blob.size();
+    static_assert(RPX_LDS_LISTS * sizeof(rpx_face_list_t) + RPX_LDS_FACES * sizeof(rpx_face_t) <= RPX_LDS_SCENE,
+                  "face lists and faces always fit");
+    size_t o_s, o_m;
+    int32_t stage_ops = -1, stage_materials = -1;
+    if (fixed + ops_bytes + mat_bytes <= RPX_LDS_SCENE || fixed + mat_bytes > RPX_LDS_SCENE) {
+        o_s = append(d->shape_ops, ops_bytes);
+        if (blob.size() <= RPX_LDS_SCENE) stage_ops = (int32_t)o_s;
+        o_m = append(d->materials, mat_bytes);
+        if (blob.size() <= RPX_LDS_SCENE) stage_materials = (int32_t)o_m;
+    } else {
+        o_m = append(d->materials, mat_bytes);
+        stage_materials = (int32_t)o_m;
+        o_s = append(d->shape_ops, ops_bytes);
+    }
+    const size_t staged = std::max(fixed, std::max(stage_ops < 0 ? 0 : stage_ops + ops_bytes,
+                                                   stage_materials < 0 ? 0 : stage_materials + mat_bytes));
     size_t o_v = push_table(blob, d->vertices, 2 * d->n_vertices);
     std::vector<ZTable> ztables;
     std::vector<ZGroup> zgroups;
@@ -328,6 +355,9 @@ extern "C" rpx_status_t rpx_scene_create(const rpx_scene_desc_t *d, rpx_scene_t 
     int nlist = 0, maxc = 0, nglob = 0;
     for (int l = 0; l < d->n_face_lists; ++l) nlist += d->face_lists[l].n_faces;
     v.n_list_faces = nlist;
+    v.stage_units = (int32_t)(staged / 16);
+    v.stage_ops = stage_ops;
+    v.stage_materials = stage_materials;
     for (int i = 0; i < nlist; ++i) {
         const rpx_face_t &f = d->faces[i];
         if (f.global_idx + 1 > nglob) nglob = f.global_idx + 1;
@@ -399,6 +429,7 @@ struct TraceArgs {
     GenLink *link;
     uint64_t pool_rays;
     int32_t in_pool, store_children;
+    int32_t count_children = 1;   // 0: the last generation of a chain whose children nobody asks for
     uint64_t status_tag;     // look-back tag of this generation (0 outside a chain)
     GenControl *head_out;    // chain: where the last workgroup to finish writes the control head
     // tile order (k_generation): with by_launch, tile = tile_base +
@@ -494,7 +525,7 @@ __global__ __launch_bounds__(RPX_BLOCK) void k_gausslet_generation(TraceArgs A) 
         if (threadIdx.x == 0) my_tile = atomicAdd(&A.ws.ctl->tile_counter, 1u);
     }
     const SceneView S = stage_scene(A.S, lds_scene);
-    for (int k = threadIdx.x; k < RPX_LDS_FACES; k += blockDim.x) lds_hist[k] = 0;
+    if (threadIdx.x < RPX_LDS_FACES) lds_hist[threadIdx.x] = 0;
     if (threadIdx.x == 0) {
         lds_tile = my_tile;
         lds_hits = 0;
@@ -545,7 +576,7 @@ __global__ __launch_bounds__(RPX_BLOCK) void k_gausslet_generation(TraceArgs A) 
                     para_ok = false;
                 }
             }
-            if (para_ok && fc.material >= 0) {
+            if (para_ok && A.count_children && fc.material >= 0) {
                 Ray r = load_ray(in, i);
                 r.length = length;
                 r.end_face_idx = end_face;
@@ -676,20 +707,23 @@ void k_generation(TraceArgs A) {
         // the scene staging
         if (threadIdx.x == 0) my_tile = atomicAdd(&A.ws.ctl->tile_counter, 1u);
     }
-    // with launch-order tiles the ray's geometry is loaded before the scene
-    // is staged, so that the two latencies overlap
+    // with launch-order tiles the ray's geometry and wavelength index are
+    // loaded before the scene is staged, so that the latencies overlap
     const double *f = in.f64;
     const uint64_t c = in.capacity;
     V3 origin = v3(0, 0, 0), dir = v3(0, 0, 0);
+    uint32_t wl_idx = 0;
+    auto load_geometry = [&](uint64_t i) {
+        origin = v3(f[RPX_OX * c + i], f[RPX_OY * c + i], f[RPX_OZ * c + i]);
+        dir = v3(f[RPX_DX * c + i], f[RPX_DY * c + i], f[RPX_DZ * c + i]);
+        wl_idx = in.u32[RPX_WL_IDX * c + i];
+    };
     if (A.by_launch) {
         const uint64_t i0 = (uint64_t)my_tile * RPX_BLOCK + threadIdx.x;
-        if (i0 < n_in) {
-            origin = v3(f[RPX_OX * c + i0], f[RPX_OY * c + i0], f[RPX_OZ * c + i0]);
-            dir = v3(f[RPX_DX * c + i0], f[RPX_DY * c + i0], f[RPX_DZ * c + i0]);
-        }
+        if (i0 < n_in) load_geometry(i0);
     }
     const SceneView S = stage_scene(A.S, lds_scene);
-    for (int k = threadIdx.x; k < RPX_LDS_FACES; k += blockDim.x) lds_hist[k] = 0;
+    if (threadIdx.x < RPX_LDS_FACES) lds_hist[threadIdx.x] = 0;
     if (threadIdx.x == 0) {
         lds_tile = my_tile;
         lds_hits = 0;
@@ -700,11 +734,11 @@ void k_generation(TraceArgs A) {
     PairEmit ce;
     bool hit = false;
     int hit_rec = -1, hit_list = -1;
+    const bool children = A.count_children;
     if (i < n_in) {
-        if (!A.by_launch) {
-            origin = v3(f[RPX_OX * c + i], f[RPX_OY * c + i], f[RPX_OZ * c + i]);
-            dir = v3(f[RPX_DX * c + i], f[RPX_DY * c + i], f[RPX_DZ * c + i]);
-        }
+        if (!A.by_launch) load_geometry(i);
+        // the wavelength arrives while the faces are searched
+        WlOne wavelength{children ? A.wavelengths[wl_idx] : 0.0};
         const NearHit nh = nearest_face<F, F != V_ALL>(S, A.S.faces, origin, dir, A.max_length, A.max_length,
                                                        A.one_list, A.one_face);
         const double length = nh.length;
@@ -716,61 +750,68 @@ void k_generation(TraceArgs A) {
         if (hit_rec >= 0) {
             atomicAdd(&lds_hist[hit_rec], 1u);
             const rpx_face_t &fc = S.faces[hit_rec];
-            if (fc.material >= 0 && material_emits(S.materials[fc.material])) {
+            if (children && fc.material >= 0 && material_emits(S.materials[fc.material])) {
                 hit = true;   // counted: the rest of its record is read
                 const rpx_face_list_t &fl = S.face_lists[hit_list];
-                Ray r = load_ray(in, i);
+                Ray r = load_ray_rest(in, i);
+                r.origin = origin;
+                r.direction = dir;
+                r.wl_idx = wl_idx;
                 r.length = length;
                 r.end_face_idx = end_face;
-                V3 hp = add(r.origin, mul(r.direction, length));
+                V3 hp = add(origin, mul(dir, length));
                 Orientation o = compute_orientation<F>(S, fl, fc, hp);
-                eval_children<F>(S.materials[fc.material], r, (uint32_t)i, hp, o, A.wavelengths, ce);
+                eval_children<F>(S.materials[fc.material], r, (uint32_t)i, hp, o, wavelength, ce);
             }
         }
     }
-    // a multi-order grating (all-features variant only) can have a third child
-    const uint32_t count = (uint32_t)min(ce.n, (F & M_GRATING) ? 3 : 2);
-    uint32_t block_total;
-    const uint32_t local = block_scan_small(count, lds_wave, &block_total);
-    {
-        const uint64_t mh = __ballot(hit);
-        if ((threadIdx.x & 63) == 0) atomicAdd(&lds_hits, (uint32_t)__popcll(mh));
-    }
-    if (threadIdx.x < 64) {
-        const uint64_t excl = lookback_tagged(A.ws.tile_status, tile, 0, block_total, &A.ws.ctl->error, A.status_tag,
-                                              A.lookback_ticks);
-        if (threadIdx.x == 0) lds_excl = excl;
-    }
-    __syncthreads();
-    const uint64_t pos = lds_excl + local;
-    if (count > 0 && pos < out_limit) store_ray(out, pos, ce.first());
-    if (count > 1 && pos + 1 < out_limit) store_ray(out, pos + 1, ce.second());
-    if constexpr ((F & M_GRATING) != 0) {
-        if (count > 2 && pos + 2 < out_limit) {
-            // the third child is built again now that its position is known
-            const rpx_face_t &fc = S.faces[hit_rec];
-            Ray r = load_ray(in, i);
-            V3 hp = add(r.origin, mul(r.direction, r.length));
-            Orientation o = compute_orientation<F>(S, S.face_lists[hit_list], fc, hp);
-            TailEmit te{&out, pos, out_limit};
-            grating_children(S.materials[fc.material], r, (uint32_t)i, hp, o, A.wavelengths, te);
+    if (children) {
+        // a multi-order grating (all-features variant only) can have a third child
+        const uint32_t count = (uint32_t)min(ce.n, (F & M_GRATING) ? 3 : 2);
+        uint32_t block_total;
+        const uint32_t local = block_scan_small(count, lds_wave, &block_total);
+        {
+            const uint64_t mh = __ballot(hit);
+            if ((threadIdx.x & 63) == 0) atomicAdd(&lds_hits, (uint32_t)__popcll(mh));
         }
-    }
-    if (threadIdx.x == 0) {
-        // a chain's hit total is the sum of its face totals (k_chain_fold);
-        // one word per generation would take every tile's atomic in one line
-        if (!A.link) add_hits(A.ws.ctl, tile, lds_hits);
-        if ((uint64_t)tile == (n_in - 1) / RPX_BLOCK) {
-            const uint64_t kids = lds_excl + block_total;
-            A.ws.ctl->children = kids;
-            if (A.link) {
-                const uint64_t at = A.link[0].out_offset;
-                A.link[1].count = kids;
-                A.link[1].offset = at;
-                A.link[1].out_offset = at + kids;
-                A.head_out->children = kids;   // host-mapped: read once the generation has ended
+        if (threadIdx.x < 64) {
+            const uint64_t excl = lookback_tagged(A.ws.tile_status, tile, 0, block_total, &A.ws.ctl->error, A.status_tag,
+                                                  A.lookback_ticks);
+            if (threadIdx.x == 0) lds_excl = excl;
+        }
+        __syncthreads();
+        const uint64_t pos = lds_excl + local;
+        if (count > 0 && pos < out_limit) store_ray(out, pos, ce.first());
+        if (count > 1 && pos + 1 < out_limit) store_ray(out, pos + 1, ce.second());
+        if constexpr ((F & M_GRATING) != 0) {
+            if (count > 2 && pos + 2 < out_limit) {
+                // the third child is built again now that its position is known
+                const rpx_face_t &fc = S.faces[hit_rec];
+                Ray r = load_ray(in, i);
+                V3 hp = add(r.origin, mul(r.direction, r.length));
+                Orientation o = compute_orientation<F>(S, S.face_lists[hit_list], fc, hp);
+                TailEmit te{&out, pos, out_limit};
+                grating_children(S.materials[fc.material], r, (uint32_t)i, hp, o, A.wavelengths, te);
             }
         }
+        if (threadIdx.x == 0) {
+            // a chain's hit total is the sum of its face totals (k_chain_fold);
+            // one word per generation would take every tile's atomic in one line
+            if (!A.link) add_hits(A.ws.ctl, tile, lds_hits);
+            if ((uint64_t)tile == (n_in - 1) / RPX_BLOCK) {
+                const uint64_t kids = lds_excl + block_total;
+                A.ws.ctl->children = kids;
+                if (A.link) {
+                    const uint64_t at = A.link[0].out_offset;
+                    A.link[1].count = kids;
+                    A.link[1].offset = at;
+                    A.link[1].out_offset = at + kids;
+                    A.head_out->children = kids;   // host-mapped: read once the generation has ended
+                }
+            }
+        }
+    } else {
+        __syncthreads();   // lds_hist is complete
     }
     if (A.face_hits || A.link) {
         uint32_t *shard = A.ws.ctl->face_shards[tile % RPX_SHARDS];
@@ -1044,11 +1085,11 @@ extern "C" uint64_t rpx_chain_workspace_bytes(uint64_t max_rays_per_generation, 
 
 // rpx_trace_rays: the float64 generations of trace_rays as one device-
 // resident chain (run_chain in rpx_gen.h).
-extern "C" rpx_status_t rpx_trace_rays(const rpx_scene_t *scene, const rpx_rays_t *in, uint64_t n_in,
-                                       float max_length, const double *wavelengths, uint64_t n_wavelengths,
-                                       int32_t max_generations, rpx_rays_t *pool, uint64_t *counts,
-                                       uint64_t *offsets, int32_t *n_traced, uint32_t *face_hits,
-                                       void *workspace, uint64_t workspace_bytes, void *stream_) {
+static rpx_status_t trace_rays_impl(const rpx_scene_t *scene, const rpx_rays_t *in, uint64_t n_in, float max_length,
+                                    const double *wavelengths, uint64_t n_wavelengths, int32_t max_generations,
+                                    rpx_rays_t *pool, uint64_t *counts, uint64_t *offsets, int32_t *n_traced, uint32_t
+                                    *face_hits, void *workspace, uint64_t workspace_bytes, void *stream_, bool
+                                    count_last) {
     if (!n_traced || !counts || !offsets) return set_error(RPX_E_INVALID, "counts / offsets / n_traced are null");
     *n_traced = 0;
     counts[0] = n_in;
@@ -1069,6 +1110,7 @@ extern "C" rpx_status_t rpx_trace_rays(const rpx_scene_t *scene, const rpx_rays_
     spec.bytes_in = 48.0 + 12.0;    // geometry read, length + end face written
     spec.bytes_hit = 100.0;         // the rest of a ray that hit
     spec.bytes_child = 188.0;       // a child record
+    spec.count_last = count_last;
     if (rpx_status_t st = check_chain(spec, scene, workspace, workspace_bytes)) return st;
     const uint32_t variant = scene_variant(scene);
     TraceArgs A;
@@ -1095,6 +1137,7 @@ extern "C" rpx_status_t rpx_trace_rays(const rpx_scene_t *scene, const rpx_rays_
         A.in_pool = cg.in_pool;
         A.in = cg.in_pool ? *pool : *in;
         A.store_children = cg.store_children;
+        A.count_children = cg.count_children;
         A.tile_base = cg.tile_base;
         A.by_launch = cg.by_launch;
         A.lookback_ticks = cg.lookback_ticks;
@@ -1104,13 +1147,32 @@ extern "C" rpx_status_t rpx_trace_rays(const rpx_scene_t *scene, const rpx_rays_
     return run_chain(spec, scene, workspace, launch, counts, offsets, n_traced, face_hits, (hipStream_t)stream_);
 }
 
+extern "C" rpx_status_t rpx_trace_rays(const rpx_scene_t *scene, const rpx_rays_t *in, uint64_t n_in, float
+                                       max_length, const double *wavelengths, uint64_t n_wavelengths, int32_t
+                                       max_generations, rpx_rays_t *pool, uint64_t *counts, uint64_t *offsets, int32_t
+                                       *n_traced, uint32_t *face_hits, void *workspace, uint64_t workspace_bytes, void
+                                       *stream_) {
+    return trace_rays_impl(scene, in, n_in, max_length, wavelengths, n_wavelengths, max_generations, pool, counts,
+                           offsets, n_traced, face_hits, workspace, workspace_bytes, stream_, true);
+}
+
+extern "C" rpx_status_t rpx_trace_rays_discard(const rpx_scene_t *scene, const rpx_rays_t *in, uint64_t n_in, float
+                                               max_length, const double *wavelengths, uint64_t n_wavelengths, int32_t
+                                               max_generations, rpx_rays_t *pool, uint64_t *counts, uint64_t *offsets,
+                                               int32_t *n_traced, uint32_t *face_hits, void *workspace, uint64_t
+                                               workspace_bytes, void *stream_) {
+    return trace_rays_impl(scene, in, n_in, max_length, wavelengths, n_wavelengths, max_generations, pool, counts,
+                           offsets, n_traced, face_hits, workspace, workspace_bytes, stream_, false);
+}
+
+
 // rpx_trace_gausslets: the gausslet generations of trace_rays as one
 // device-resident chain (run_chain in rpx_gen.h).
-extern "C" rpx_status_t rpx_trace_gausslets(const rpx_scene_t *scene, const rpx_rays_t *in, uint64_t n_in,
-                                       double max_length, const double *wavelengths, uint64_t n_wavelengths,
-                                       int32_t max_generations, rpx_rays_t *pool, uint64_t *counts,
-                                       uint64_t *offsets, int32_t *n_traced, uint32_t *face_hits,
-                                       void *workspace, uint64_t workspace_bytes, void *stream_) {
+static rpx_status_t trace_gausslets_impl(const rpx_scene_t *scene, const rpx_rays_t *in, uint64_t n_in, double
+                                         max_length, const double *wavelengths, uint64_t n_wavelengths, int32_t
+                                         max_generations, rpx_rays_t *pool, uint64_t *counts, uint64_t *offsets,
+                                         int32_t *n_traced, uint32_t *face_hits, void *workspace, uint64_t
+                                         workspace_bytes, void *stream_, bool count_last) {
     if (!n_traced || !counts || !offsets) return set_error(RPX_E_INVALID, "counts / offsets / n_traced are null");
     *n_traced = 0;
     counts[0] = n_in;
@@ -1137,6 +1199,7 @@ extern "C" rpx_status_t rpx_trace_gausslets(const rpx_scene_t *scene, const rpx_
     spec.bytes_hit = 100.0 + 6 * 32.0;
     spec.bytes_child = 188.0 + 6 * 80.0;
     spec.bytes_per_parent = true;
+    spec.count_last = count_last;
     if (rpx_status_t st = check_chain(spec, scene, workspace, workspace_bytes)) return st;
     const uint32_t variant = scene_variant(scene);
     TraceArgs A;
@@ -1163,6 +1226,7 @@ extern "C" rpx_status_t rpx_trace_gausslets(const rpx_scene_t *scene, const rpx_
         A.in_pool = cg.in_pool;
         A.in = cg.in_pool ? *pool : *in;
         A.store_children = cg.store_children;
+        A.count_children = cg.count_children;
         A.tile_base = cg.tile_base;
         A.by_launch = cg.by_launch;
         A.lookback_ticks = cg.lookback_ticks;
@@ -1171,6 +1235,26 @@ extern "C" rpx_status_t rpx_trace_gausslets(const rpx_scene_t *scene, const rpx_
     };
     return run_chain(spec, scene, workspace, launch, counts, offsets, n_traced, face_hits, (hipStream_t)stream_);
 }
+
+extern "C" rpx_status_t rpx_trace_gausslets(const rpx_scene_t *scene, const rpx_rays_t *in, uint64_t n_in, double
+                                            max_length, const double *wavelengths, uint64_t n_wavelengths, int32_t
+                                            max_generations, rpx_rays_t *pool, uint64_t *counts, uint64_t *offsets,
+                                            int32_t *n_traced, uint32_t *face_hits, void *workspace, uint64_t
+                                            workspace_bytes, void *stream_) {
+    return trace_gausslets_impl(scene, in, n_in, max_length, wavelengths, n_wavelengths, max_generations, pool,
+                                counts, offsets, n_traced, face_hits, workspace, workspace_bytes, stream_, true);
+}
+
+extern "C" rpx_status_t rpx_trace_gausslets_discard(const rpx_scene_t *scene, const rpx_rays_t *in, uint64_t n_in,
+                                                    double max_length, const double *wavelengths, uint64_t
+                                                    n_wavelengths, int32_t max_generations, rpx_rays_t *pool, uint64_t
+                                                    *counts, uint64_t *offsets, int32_t *n_traced, uint32_t
+                                                    *face_hits, void *workspace, uint64_t workspace_bytes, void
+                                                    *stream_) {
+    return trace_gausslets_impl(scene, in, n_in, max_length, wavelengths, n_wavelengths, max_generations, pool,
+                                counts, offsets, n_traced, face_hits, workspace, workspace_bytes, stream_, false);
+}
+
 
 // ------------------------------------------------------ AoS <-> SoA
 // Packed ray_t: 21 doubles (168 B) then 5 uint32 (20 B) = 188 B = 47 words.

@@ -174,7 +174,7 @@ def _split_generation(ctx, rays, max_length, one_list=-1, one_face=-1):
 
 
 def _split_chain(ctx, rays, max_length, limit):
-    """The FP32-split generations on the device (rpx_trace_rays_split), with
+    """The FP32-split generations on the device (rpx_trace_rays_split_discard), with
     the pool and resume bookkeeping of tracer._trace_chain."""
     from .tracer import _pool_rays, _alloc_pool
     lib = load()
@@ -192,10 +192,11 @@ def _split_chain(ctx, rays, max_length, limit):
         offsets = (ctypes.c_uint64 * (remaining + 1))()
         n_traced = ctypes.c_int32(0)
         s_in, s_pool = current.dev.struct(), pool.struct()
-        code = lib.rpx_trace_rays_split(ctx.handle, ctypes.byref(s_in), n, float(max_length),
-                                        ctypes.c_void_p(current._wl_dev.data_ptr()), len(current._wavelengths),
-                                        remaining, ctypes.byref(s_pool), counts, offsets, ctypes.byref(n_traced),
-                                        hits, ctypes.c_void_p(ws.data_ptr()), ws_bytes, stream_handle())
+        code = lib.rpx_trace_rays_split_discard(ctx.handle, ctypes.byref(s_in), n, float(max_length),
+                                                ctypes.c_void_p(current._wl_dev.data_ptr()), len(current._wavelengths),
+                                                remaining, ctypes.byref(s_pool), counts, offsets,
+                                                ctypes.byref(n_traced),
+                                                hits, ctypes.c_void_p(ws.data_ptr()), ws_bytes, stream_handle())
         if code != _abi.RPX_E_CAPACITY:
             check(code)
         k_traced = n_traced.value
@@ -222,7 +223,7 @@ def _split_chain(ctx, rays, max_length, limit):
 def trace_rays_split(input_rays, face_lists, recursion_limit=100, max_length=100.0):
     """FP32-split non-sequential trace of a RayCollection; generation
     bookkeeping as tracer.trace_rays (core/tracer.py:9-47).  The generations
-    run device-resident (rpx_trace_rays_split), which writes every input
+    run device-resident (rpx_trace_rays_split_discard), which writes every input
     ray's length itself."""
     all_faces = _prepare(input_rays, face_lists, max_length, reset=False)
     face_sets = list(face_lists)

@@ -92,8 +92,8 @@ def _alloc_pool(make, want, minimum):
 
 
 def _trace_chain(ctx, rays, max_length, limit):
-    """trace_rays' generation loop for a RayCollection (rpx_trace_rays) or a
-    GaussletCollection (rpx_trace_gausslets) on the device: generations are
+    """trace_rays' generation loop for a RayCollection (rpx_trace_rays_discard) or a
+    GaussletCollection (rpx_trace_gausslets_discard) on the device: generations are
     written into pools and traced with no host round trip between them; a
     pool that cannot be sure to hold the next generation ends the call, and
     the loop continues from that generation with a fresh pool.  Returns the
@@ -103,7 +103,7 @@ def _trace_chain(ctx, rays, max_length, limit):
     lib = load()
     gauss = isinstance(rays, GaussletCollection)
     cls = GaussletCollection if gauss else RayCollection
-    entry = lib.rpx_trace_gausslets if gauss else lib.rpx_trace_rays
+    entry = lib.rpx_trace_gausslets_discard if gauss else lib.rpx_trace_rays_discard
     traced = [rays]
     current = rays
     remaining = limit
