@@ -4,7 +4,7 @@
 // traces the current generation of all active jobs together, and then up to
 // three more without a host round trip (each laid out on the device from
 // the previous one's child counts, k_batch_relayout): the jobs' rays are
-// laid end to end as tiles of RPX_BLOCK rays, and one launch of one
+// laid end to end as tiles of 256 or 512 rays, and one launch of one
 // workgroup per tile takes tile numbers from an atomic counter.  A workgroup
 // stages the scene of the job its tile belongs to in LDS, traces the tile as
 // k_generation does (same face, orientation and material code), places the
@@ -69,7 +69,16 @@ struct BatchControl {
     uint64_t error;
     uint32_t tile_counter;
     uint32_t next_block;             // the generation of the step the next relayout lays out (1, 2, ...)
+    uint32_t tile_rays;              // rays per tile of this step (BATCH_SMALL or BATCH_LARGE)
+    uint32_t pad;
 };
+
+// Rays per tile of a step: as the chains' (gen_block in rpx_trace.hip), 512 for
+// the lens variants in steps of at least 65,536 rays (24 lens jobs of up to
+// 500,000 rays: 282 -> 235 us per tile kernel), else 256.  Moment partials are
+// kept per 256 rays either way, so that a job's sums do not depend on the size.
+#define BATCH_SMALL 256
+#define BATCH_LARGE 512
 
 // Generations one server step can trace per job, and the count words each
 // generation of a step has per job.
@@ -96,7 +105,8 @@ __global__ __launch_bounds__(256) void k_batch_reduce(const BatchJob *jobs, cons
     if (j >= ctl->n_jobs) return;
     const BatchJob &J = jobs[j];
     double s[5] = {0, 0, 0, 0, 0};
-    for (uint64_t t = J.tile_begin + threadIdx.x; t < J.tile_end; t += 256)
+    const uint64_t parts = ctl->tile_rays / BATCH_SMALL;
+    for (uint64_t t = J.tile_begin * parts + threadIdx.x; t < J.tile_end * parts; t += 256)
         for (int q = 0; q < 5; ++q) s[q] += partials[t * 5 + q];
     for (int q = 0; q < 5; ++q) red[threadIdx.x][q] = s[q];
     __syncthreads();
@@ -122,6 +132,7 @@ __global__ __launch_bounds__(256) void k_batch_relayout(BatchJob *jobs, BatchCon
     __shared__ uint64_t run_tiles[256];
     const uint32_t n = (uint32_t)ctl->n_jobs;
     const uint32_t blk = ctl->next_block;
+    const uint64_t B = ctl->tile_rays;
     const uint32_t per = (n + 255) / 256;
     const uint32_t b = threadIdx.x * per, e = min(n, b + per);
     auto traces = [blk](const BatchJob &J, uint64_t kids) {
@@ -130,7 +141,7 @@ __global__ __launch_bounds__(256) void k_batch_relayout(BatchJob *jobs, BatchCon
     uint64_t mine = 0;
     for (uint32_t j = b; j < e; ++j) {
         const uint64_t kids = jobs[j].counts[0];
-        if (traces(jobs[j], kids)) mine += (kids + RPX_BLOCK - 1) / RPX_BLOCK;
+        if (traces(jobs[j], kids)) mine += (kids + B - 1) / B;
     }
     run_tiles[threadIdx.x] = mine;
     __syncthreads();
@@ -145,7 +156,7 @@ __global__ __launch_bounds__(256) void k_batch_relayout(BatchJob *jobs, BatchCon
         J.out = first_in;
         J.n_in = go ? kids : 0;
         J.tile_begin = base;
-        base += go ? (kids + RPX_BLOCK - 1) / RPX_BLOCK : 0;
+        base += go ? (kids + B - 1) / B : 0;
         J.tile_end = base;
         J.counts += 4;
         J.counts[3] = go ? 1 : 0;
@@ -157,16 +168,16 @@ __global__ __launch_bounds__(256) void k_batch_relayout(BatchJob *jobs, BatchCon
     }
 }
 
-template <uint32_t F>
-__global__ __launch_bounds__(RPX_BLOCK) __attribute__((amdgpu_waves_per_eu(F == V_ALL ? 3 : 4)))
+template <uint32_t F, int B>
+__global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(F == V_ALL ? 3 : 4)))
 void k_batch(const BatchJob *jobs, BatchControl *ctl, uint64_t *status,
                                                      double *partials) {
     __shared__ SceneLds lds_scene;
-    __shared__ uint32_t lds_wave[RPX_BLOCK / 64];
+    __shared__ uint32_t lds_wave[B / 64];
     __shared__ uint64_t lds_tile, lds_excl;
     __shared__ int32_t lds_job;
     __shared__ uint32_t lds_parents, lds_hits;
-    __shared__ double lds_mom[RPX_BLOCK / 64][5];
+    __shared__ double lds_mom[B / 64][5];
     const uint64_t total = ctl->total_tiles;
     const int n_jobs = (int)ctl->n_jobs;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -195,7 +206,7 @@ void k_batch(const BatchJob *jobs, BatchControl *ctl, uint64_t *status,
         const BatchJob &J = jobs[j];
         const SceneView S = stage_scene(J.S, lds_scene);
         __syncthreads();
-        const uint64_t i = (tile - J.tile_begin) * RPX_BLOCK + threadIdx.x;
+        const uint64_t i = (tile - J.tile_begin) * B + threadIdx.x;
         PairEmit ce;
         bool hit = false;
         double mx = 0, my = 0, mz = 0, mr = 0, mn = 0;
@@ -264,11 +275,12 @@ void k_batch(const BatchJob *jobs, BatchControl *ctl, uint64_t *status,
             if (lds_hits) atomicAdd((unsigned long long *)&J.counts[1], (unsigned long long)lds_hits);
             if (lds_parents) atomicAdd((unsigned long long *)&J.counts[2], (unsigned long long)lds_parents);
             if (tile == J.tile_end - 1) J.counts[0] = lds_excl + block_total;
-            for (int q = 0; q < 5; ++q) {
-                double v = 0;
-                for (int w = 0; w < RPX_BLOCK / 64; ++w) v += lds_mom[w][q];
-                partials[tile * 5 + q] = v;
-            }
+        }
+        if (threadIdx.x < 5 * (B / BATCH_SMALL)) {
+            const int part = threadIdx.x / 5, q = threadIdx.x % 5;
+            double v = 0;
+            for (int w = 0; w < BATCH_SMALL / 64; ++w) v += lds_mom[part * (BATCH_SMALL / 64) + w][q];
+            partials[(tile * (B / BATCH_SMALL) + part) * 5 + q] = v;
         }
     }
 }
@@ -317,6 +329,7 @@ struct StepGraph {
     int gens = 0;                                        // generations the graph traces
     hipGraphNode_t clear[RPX_SERVE_MAX_GENS] = {}, batch[RPX_SERVE_MAX_GENS] = {};
     void *batch_func = nullptr;
+    unsigned batch_block = BATCH_SMALL;
 };
 
 struct rpx_server {
@@ -332,7 +345,7 @@ struct rpx_server {
     double *d_partials = nullptr;
     uint64_t *d_counts = nullptr, *h_counts = nullptr;
     double *d_moments = nullptr, *h_moments = nullptr;
-    StepGraph graphs[RPX_SERVE_MAX_GENS][3];   // by generations per step - 1, then kernel variant
+    StepGraph graphs[RPX_SERVE_MAX_GENS][5];   // by generations per step - 1, then kernel instance
     uint32_t gens_per_step = 2;
     bool graph_launch = true;    // replay the step graph (else launch its nodes one by one)
     void *clear_args[4] = {&d_status, &max_tiles, &d_jobs, &d_ctl};
@@ -378,7 +391,7 @@ static void free_buffer(rpx_server_t *s, Buffer &b) {
                                                                    hipGetErrorString(_e));    \
     } while (0)
 
-template <uint32_t F>
+template <uint32_t F, int B>
 static rpx_status_t build_graph(rpx_server_t *s, StepGraph &G, int gens) {
     RPX_GRAPH_TRY(hipGraphCreate(&G.g, 0));
     hipGraphNode_t last, node;
@@ -407,7 +420,7 @@ static rpx_status_t build_graph(rpx_server_t *s, StepGraph &G, int gens) {
         if (k > 0)
             RPX_GRAPH_TRY(add_kernel((void *)k_batch_relayout, dim3(1), dim3(256), s->relayout_args, nullptr));
         RPX_GRAPH_TRY(add_kernel((void *)k_batch_clear, dim3(1), dim3(256), s->clear_args, &G.clear[k]));
-        RPX_GRAPH_TRY(add_kernel((void *)k_batch<F>, dim3(1), dim3(RPX_BLOCK), s->batch_args, &G.batch[k]));
+        RPX_GRAPH_TRY(add_kernel((void *)k_batch<F, B>, dim3(1), dim3(B), s->batch_args, &G.batch[k]));
         RPX_GRAPH_TRY(add_kernel((void *)k_batch_reduce, dim3(s->max_jobs), dim3(256), s->reduce_args, nullptr));
     }
     G.gens = gens;
@@ -421,7 +434,8 @@ static rpx_status_t build_graph(rpx_server_t *s, StepGraph &G, int gens) {
     RPX_GRAPH_TRY(hipGraphAddMemcpyNode1D(&node, G.g, &last, 1, s->h_ctl_back, s->d_ctl, sizeof(BatchControl),
                                           hipMemcpyDeviceToHost));
     RPX_GRAPH_TRY(hipGraphInstantiate(&G.exec, G.g, nullptr, nullptr, 0));
-    G.batch_func = (void *)k_batch<F>;
+    G.batch_func = (void *)k_batch<F, B>;
+    G.batch_block = B;
     return RPX_OK;
 }
 
@@ -438,7 +452,7 @@ static rpx_status_t size_graph(rpx_server_t *s, StepGraph &G, const uint64_t *ti
         RPX_GRAPH_TRY(hipGraphExecKernelNodeSetParams(G.exec, clear, &p));
         p.func = G.batch_func;
         p.gridDim = dim3((unsigned)std::max<uint64_t>(t, 1));
-        p.blockDim = dim3(RPX_BLOCK);
+        p.blockDim = dim3(G.batch_block);
         p.kernelParams = s->batch_args;
         RPX_GRAPH_TRY(hipGraphExecKernelNodeSetParams(G.exec, batch, &p));
         return RPX_OK;
@@ -452,7 +466,7 @@ static rpx_status_t size_graph(rpx_server_t *s, StepGraph &G, const uint64_t *ti
 // job table (only the batched jobs' entries) and control block up, per
 // generation the relayout (after the first), clear, tile kernel and moment
 // sums, then the counts, moments and control block back.
-template <uint32_t F>
+template <uint32_t F, int B>
 static rpx_status_t launch_step(rpx_server_t *s, int gens, const uint64_t *tiles, uint64_t n_jobs) {
     hipStream_t st = s->stream;
     RPX_HIP_TRY(hipMemcpyAsync(s->d_jobs, s->h_jobs, sizeof(BatchJob) * n_jobs, hipMemcpyHostToDevice, st));
@@ -462,7 +476,7 @@ static rpx_status_t launch_step(rpx_server_t *s, int gens, const uint64_t *tiles
         const uint64_t t = tiles[k];
         hipLaunchKernelGGL(k_batch_clear, dim3((unsigned)((std::max(t, n_jobs) + 255) / 256)), dim3(256), 0, st,
                            s->d_status, s->max_tiles, s->d_jobs, s->d_ctl);
-        hipLaunchKernelGGL((k_batch<F>), dim3((unsigned)std::max<uint64_t>(t, 1)), dim3(RPX_BLOCK), 0, st,
+        hipLaunchKernelGGL((k_batch<F, B>), dim3((unsigned)std::max<uint64_t>(t, 1)), dim3(B), 0, st,
                            s->d_jobs, s->d_ctl, s->d_status, s->d_partials);
         hipLaunchKernelGGL(k_batch_reduce, dim3((unsigned)n_jobs), dim3(256), 0, st, s->d_jobs, s->d_ctl,
                            s->d_partials);
@@ -489,7 +503,7 @@ extern "C" rpx_status_t rpx_server_create(uint64_t hbm_budget_bytes, uint32_t ma
     s->budget = hbm_budget_bytes;
     s->heap.set_limits(hbm_budget_bytes, std::min<uint64_t>(hbm_budget_bytes, 256ull << 20));
     s->max_jobs = max_jobs;
-    s->max_tiles = (max_rays_in_flight + RPX_BLOCK - 1) / RPX_BLOCK + max_jobs;
+    s->max_tiles = (max_rays_in_flight + BATCH_SMALL - 1) / BATCH_SMALL + max_jobs;
     auto fail = [&](rpx_status_t st) {
         rpx_server_destroy(s);
         return st;
@@ -499,7 +513,7 @@ extern "C" rpx_status_t rpx_server_create(uint64_t hbm_budget_bytes, uint32_t ma
     if (hipMalloc(&s->d_jobs, sizeof(BatchJob) * max_jobs) != hipSuccess ||
         hipMalloc(&s->d_ctl, sizeof(BatchControl)) != hipSuccess ||
         hipMalloc(&s->d_status, sizeof(uint64_t) * s->max_tiles) != hipSuccess ||
-        hipMalloc(&s->d_partials, sizeof(double) * 5 * s->max_tiles) != hipSuccess ||
+        hipMalloc(&s->d_partials, sizeof(double) * 5 * (s->max_tiles + max_jobs)) != hipSuccess ||
         hipMalloc(&s->d_counts, sizeof(uint64_t) * RPX_SERVE_COUNT_WORDS * max_jobs) != hipSuccess ||
         hipMalloc(&s->d_moments, sizeof(double) * 6 * max_jobs) != hipSuccess ||
         hipHostMalloc(&s->h_jobs, sizeof(BatchJob) * max_jobs, 0) != hipSuccess ||
@@ -557,7 +571,7 @@ extern "C" rpx_status_t rpx_server_submit(rpx_server_t *s, const rpx_job_desc_t 
     if (!d->rays || d->rays->capacity < d->n_rays || (d->n_rays && (!d->rays->f64 || !d->rays->u32)))
         return rpx_set_error(RPX_E_INVALID, "job rays");
     if (d->n_rays > 0xFFFFFFFFull) return rpx_set_error(RPX_E_UNSUPPORTED, "more than 2^32-1 rays in a job");
-    if ((d->n_rays + RPX_BLOCK - 1) / RPX_BLOCK + 1 > s->max_tiles)
+    if ((d->n_rays + BATCH_SMALL - 1) / BATCH_SMALL + 1 > s->max_tiles)
         return rpx_set_error(RPX_E_CAPACITY, "job larger than the server's rays in flight");
     if (d->n_wavelengths && !d->wavelengths) return rpx_set_error(RPX_E_INVALID, "wavelength table is null");
     if (d->scene->view.max_children > 2)
@@ -628,12 +642,12 @@ extern "C" rpx_status_t rpx_server_step(rpx_server_t *s, rpx_job_result_t *finis
     *n_finished = 0;
     // admission, first come first served
     uint64_t tiles_active = 0;
-    for (Job *j : s->active) tiles_active += (j->n + RPX_BLOCK - 1) / RPX_BLOCK;
+    for (Job *j : s->active) tiles_active += (j->n + BATCH_SMALL - 1) / BATCH_SMALL;
     while (!s->waiting.empty() && !s->free_slots.empty()) {
         Job *j = s->waiting.front();
         // its input is already counted; the children buffer is what it adds
         const uint64_t need = std::max<uint64_t>((uint64_t)j->max_children * j->n, 1) * RAY_BYTES;
-        const uint64_t tiles = (j->n + RPX_BLOCK - 1) / RPX_BLOCK;
+        const uint64_t tiles = (j->n + BATCH_SMALL - 1) / BATCH_SMALL;
         if (!s->active.empty() && (s->used + need > s->budget || tiles_active + tiles > s->max_tiles)) {
             if (s->used + need > s->budget && !j->held_for_budget) {
                 j->held_for_budget = true;
@@ -673,7 +687,7 @@ extern "C" rpx_status_t rpx_server_step(rpx_server_t *s, rpx_job_result_t *finis
     // a job whose generation alone exceeds the status table cannot run
     for (size_t k = 0; k < s->active.size();) {
         Job *j = s->active[k];
-        if ((j->n + RPX_BLOCK - 1) / RPX_BLOCK > s->max_tiles) {
+        if ((j->n + BATCH_SMALL - 1) / BATCH_SMALL > s->max_tiles) {
             j->status = RPX_E_CAPACITY;
             s->active.erase(s->active.begin() + k);
             finish(s, j, now_s());
@@ -685,11 +699,11 @@ extern "C" rpx_status_t rpx_server_step(rpx_server_t *s, rpx_job_result_t *finis
     // fit the status table; the others wait for the next step
     std::vector<Job *> batch;
     if (!s->active.empty()) {
-        uint64_t tile = 0;
+        uint64_t tile = 0, rays = 0;   // tiles of BATCH_SMALL, which the status table is sized for
         uint32_t variant = V_SPHERES;
         for (size_t k = 0; k < s->active.size(); ++k) {
             Job *j = s->active[k];
-            const uint64_t tiles = (j->n + RPX_BLOCK - 1) / RPX_BLOCK;
+            const uint64_t tiles = (j->n + BATCH_SMALL - 1) / BATCH_SMALL;
             if (tile + tiles > s->max_tiles) continue;
             BatchJob &b = s->h_jobs[batch.size()];
             batch.push_back(j);
@@ -697,9 +711,8 @@ extern "C" rpx_status_t rpx_server_step(rpx_server_t *s, rpx_job_result_t *finis
             b.in = j->cur.rays();
             b.out = j->next.rays();
             b.n_in = j->n;
-            b.tile_begin = tile;
             tile += tiles;
-            b.tile_end = tile;
+            rays += j->n;
             b.max_length = (double)j->desc.max_length;
             b.wl.wl = j->desc.wavelengths;
             b.wl.n = j->desc.wavelengths ? j->desc.n_wavelengths : 0;
@@ -713,6 +726,13 @@ extern "C" rpx_status_t rpx_server_step(rpx_server_t *s, rpx_job_result_t *finis
             b.counts = s->d_counts + j->slot * RPX_SERVE_COUNT_WORDS;
             if (j->variant == V_ALL || (j->variant == V_LENS && variant == V_SPHERES)) variant = j->variant;
         }
+        const uint64_t B = variant != V_ALL && rays >= 65536 ? BATCH_LARGE : BATCH_SMALL;
+        tile = 0;
+        for (size_t k = 0; k < batch.size(); ++k) {
+            s->h_jobs[k].tile_begin = tile;
+            tile += (batch[k]->n + B - 1) / B;
+            s->h_jobs[k].tile_end = tile;
+        }
         // tiles of each generation of the step: the first's exact, the later
         // ones' bounded by the buffer they are written into (the job's two
         // buffers alternate, the second generation writing into `cur`), over
@@ -725,9 +745,9 @@ extern "C" rpx_status_t rpx_server_step(rpx_server_t *s, rpx_job_result_t *finis
             for (size_t k = 0; k < batch.size(); ++k) {
                 if (s->h_jobs[k].gens <= g) continue;
                 const Buffer &into = (g % 2 == 1) ? batch[k]->cur : batch[k]->next;
-                t += (into.cap / std::max(1, batch[k]->max_children) + RPX_BLOCK - 1) / RPX_BLOCK;
+                t += (into.cap / std::max(1, batch[k]->max_children) + B - 1) / B;
             }
-            if (t == 0 || t > s->max_tiles) break;
+            if (t == 0 || t * (B / BATCH_SMALL) > s->max_tiles) break;
             tiles[g] = t;
             gens = g + 1;
         }
@@ -737,22 +757,27 @@ extern "C" rpx_status_t rpx_server_step(rpx_server_t *s, rpx_job_result_t *finis
         s->h_ctl->error = 0;
         s->h_ctl->tile_counter = 0;
         s->h_ctl->next_block = 1;
-        const int vi = variant == V_SPHERES ? 0 : variant == V_LENS ? 1 : 2;
+        s->h_ctl->tile_rays = (uint32_t)B;
+        const int vi = variant == V_ALL ? 4 : (variant == V_LENS ? 2 : 0) + (B == BATCH_LARGE ? 1 : 0);
         if (s->graph_launch) {
             StepGraph &G = s->graphs[gens - 1][vi];
             if (!G.exec) {
-                rpx_status_t st = vi == 0 ? build_graph<V_SPHERES>(s, G, gens)
-                                : vi == 1 ? build_graph<V_LENS>(s, G, gens)
-                                          : build_graph<V_ALL>(s, G, gens);
+                rpx_status_t st = vi == 0 ? build_graph<V_SPHERES, BATCH_SMALL>(s, G, gens)
+                                : vi == 1 ? build_graph<V_SPHERES, BATCH_LARGE>(s, G, gens)
+                                : vi == 2 ? build_graph<V_LENS, BATCH_SMALL>(s, G, gens)
+                                : vi == 3 ? build_graph<V_LENS, BATCH_LARGE>(s, G, gens)
+                                          : build_graph<V_ALL, BATCH_SMALL>(s, G, gens);
                 if (st) return st;
             }
             rpx_status_t st = size_graph(s, G, tiles, batch.size());
             if (st) return st;
             RPX_HIP_TRY(hipGraphLaunch(G.exec, s->stream));
         } else {
-            rpx_status_t st = vi == 0 ? launch_step<V_SPHERES>(s, gens, tiles, batch.size())
-                            : vi == 1 ? launch_step<V_LENS>(s, gens, tiles, batch.size())
-                                      : launch_step<V_ALL>(s, gens, tiles, batch.size());
+            rpx_status_t st = vi == 0 ? launch_step<V_SPHERES, BATCH_SMALL>(s, gens, tiles, batch.size())
+                            : vi == 1 ? launch_step<V_SPHERES, BATCH_LARGE>(s, gens, tiles, batch.size())
+                            : vi == 2 ? launch_step<V_LENS, BATCH_SMALL>(s, gens, tiles, batch.size())
+                            : vi == 3 ? launch_step<V_LENS, BATCH_LARGE>(s, gens, tiles, batch.size())
+                                      : launch_step<V_ALL, BATCH_SMALL>(s, gens, tiles, batch.size());
             if (st) return st;
         }
         RPX_HIP_TRY(hipStreamSynchronize(s->stream));

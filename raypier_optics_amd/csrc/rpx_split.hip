@@ -165,6 +165,7 @@ void k_generation_split(SplitArgs A) {
     bool hit = false;
     int hit_rec = -1, hit_list = -1;
     double hit_length = 0;
+    uint32_t end_face = RPX_NO_FACE;
     const bool children = A.count_children;
     if (i < n_in) {
         if (!A.by_launch) load_geometry(i);
@@ -179,11 +180,9 @@ void k_generation_split(SplitArgs A) {
         const NearHit nh = nearest_face<F, F != V_ALL>(S, A.S.faces, origin, dir, A.max_length, A.max_length,
                                                        A.one_list, A.one_face);
         const double length = nh.length;
-        const uint32_t end_face = nh.end_face;
+        end_face = nh.end_face;
         hit_rec = nh.rec;
         hit_list = nh.list;
-        in.f32[RPX_S_LENGTH * c + i] = (float)length;
-        in.u32[RPX_END_FACE_IDX * c + i] = end_face;
         hit_length = length;
         if (hit_rec >= 0) {
             atomicAdd(&lds_hist[hit_rec], 1u);
@@ -218,6 +217,11 @@ void k_generation_split(SplitArgs A) {
             if (threadIdx.x == 0) lds_excl = excl;
         }
         __syncthreads();
+        // as k_generation: no store before the last load
+        if (i < n_in) {
+            in.f32[RPX_S_LENGTH * c + i] = (float)hit_length;
+            in.u32[RPX_END_FACE_IDX * c + i] = end_face;
+        }
         const uint64_t pos = lds_excl + local;
         if (count > 0 && pos < out_limit) store_ray_s(out, pos, ce.first());
         if (count > 1 && pos + 1 < out_limit) store_ray_s(out, pos + 1, ce.second());
@@ -250,6 +254,10 @@ void k_generation_split(SplitArgs A) {
             }
         }
     } else {
+        if (i < n_in) {
+            in.f32[RPX_S_LENGTH * c + i] = (float)hit_length;
+            in.u32[RPX_END_FACE_IDX * c + i] = end_face;
+        }
         __syncthreads();   // lds_hist is complete
     }
     if (A.face_hits || A.link) {

@@ -672,13 +672,15 @@ __global__ __launch_bounds__(RPX_BLOCK) void k_gausslet_generation(TraceArgs A) 
 // library paths), and a lens generation issues 1,400-1,775 vector instructions
 // per wave where it issued 2,330.  MI355X, 4,194,304 rays of the asphere and
 // doublet: 0.61-0.66 -> 0.50-0.55 ms per generation; Michelson, 65,536 rays to
-// depth 12: 16.0 -> 12.2 ms per trace.
-template <uint32_t F>
-__global__ __launch_bounds__(RPX_BLOCK) __attribute__((amdgpu_waves_per_eu(F == V_ALL ? 3 : 4)))
+// depth 12: 16.0 -> 12.2 ms per trace.  The ray's own length and end face are
+// stored last: 2 % of a lens generation.
+// B: rays per tile (gen_block).
+template <uint32_t F, int B>
+__global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(F == V_ALL ? 3 : 4)))
 void k_generation(TraceArgs A) {
     __shared__ SceneLds lds_scene;
     __shared__ uint32_t lds_hist[RPX_LDS_FACES];
-    __shared__ uint32_t lds_wave[RPX_BLOCK / 64];
+    __shared__ uint32_t lds_wave[B / 64];
     __shared__ uint32_t lds_tile, lds_hits;
     __shared__ uint64_t lds_excl;
     // A generation of a device-resident chain learns its size and place in
@@ -696,7 +698,7 @@ void k_generation(TraceArgs A) {
         out = advance_rays(A.out, L.out_offset);
         out_limit = A.store_children ? (A.pool_rays > L.out_offset ? A.pool_rays - L.out_offset : 0) : 0;
     }
-    const uint32_t n_tiles = (uint32_t)((n_in + RPX_BLOCK - 1) / RPX_BLOCK);
+    const uint32_t n_tiles = (uint32_t)((n_in + B - 1) / B);
     uint32_t my_tile = 0;
     if (A.by_launch) {
         my_tile = A.tile_base + blockIdx.x;
@@ -719,7 +721,7 @@ void k_generation(TraceArgs A) {
         wl_idx = in.u32[RPX_WL_IDX * c + i];
     };
     if (A.by_launch) {
-        const uint64_t i0 = (uint64_t)my_tile * RPX_BLOCK + threadIdx.x;
+        const uint64_t i0 = (uint64_t)my_tile * B + threadIdx.x;
         if (i0 < n_in) load_geometry(i0);
     }
     const SceneView S = stage_scene(A.S, lds_scene);
@@ -730,10 +732,12 @@ void k_generation(TraceArgs A) {
     }
     __syncthreads();
     const uint32_t tile = lds_tile;
-    const uint64_t i = (uint64_t)tile * RPX_BLOCK + threadIdx.x;
+    const uint64_t i = (uint64_t)tile * B + threadIdx.x;
     PairEmit ce;
     bool hit = false;
     int hit_rec = -1, hit_list = -1;
+    double length = 0;
+    uint32_t end_face = RPX_NO_FACE;
     const bool children = A.count_children;
     if (i < n_in) {
         if (!A.by_launch) load_geometry(i);
@@ -741,12 +745,10 @@ void k_generation(TraceArgs A) {
         WlOne wavelength{children ? A.wavelengths[wl_idx] : 0.0};
         const NearHit nh = nearest_face<F, F != V_ALL>(S, A.S.faces, origin, dir, A.max_length, A.max_length,
                                                        A.one_list, A.one_face);
-        const double length = nh.length;
-        const uint32_t end_face = nh.end_face;
+        length = nh.length;
+        end_face = nh.end_face;
         hit_rec = nh.rec;
         hit_list = nh.list;
-        in.f64[RPX_LENGTH * c + i] = length;
-        in.u32[RPX_END_FACE_IDX * c + i] = end_face;
         if (hit_rec >= 0) {
             atomicAdd(&lds_hist[hit_rec], 1u);
             const rpx_face_t &fc = S.faces[hit_rec];
@@ -780,6 +782,12 @@ void k_generation(TraceArgs A) {
             if (threadIdx.x == 0) lds_excl = excl;
         }
         __syncthreads();
+        // the ray's own length and end face go out with the children: loads that
+        // follow a store wait for it (one counter orders both)
+        if (i < n_in) {
+            in.f64[RPX_LENGTH * c + i] = length;
+            in.u32[RPX_END_FACE_IDX * c + i] = end_face;
+        }
         const uint64_t pos = lds_excl + local;
         if (count > 0 && pos < out_limit) store_ray(out, pos, ce.first());
         if (count > 1 && pos + 1 < out_limit) store_ray(out, pos + 1, ce.second());
@@ -788,6 +796,7 @@ void k_generation(TraceArgs A) {
                 // the third child is built again now that its position is known
                 const rpx_face_t &fc = S.faces[hit_rec];
                 Ray r = load_ray(in, i);
+                r.length = length;
                 V3 hp = add(r.origin, mul(r.direction, r.length));
                 Orientation o = compute_orientation<F>(S, S.face_lists[hit_list], fc, hp);
                 TailEmit te{&out, pos, out_limit};
@@ -798,7 +807,7 @@ void k_generation(TraceArgs A) {
             // a chain's hit total is the sum of its face totals (k_chain_fold);
             // one word per generation would take every tile's atomic in one line
             if (!A.link) add_hits(A.ws.ctl, tile, lds_hits);
-            if ((uint64_t)tile == (n_in - 1) / RPX_BLOCK) {
+            if ((uint64_t)tile == (n_in - 1) / B) {
                 const uint64_t kids = lds_excl + block_total;
                 A.ws.ctl->children = kids;
                 if (A.link) {
@@ -811,6 +820,10 @@ void k_generation(TraceArgs A) {
             }
         }
     } else {
+        if (i < n_in) {
+            in.f64[RPX_LENGTH * c + i] = length;
+            in.u32[RPX_END_FACE_IDX * c + i] = end_face;
+        }
         __syncthreads();   // lds_hist is complete
     }
     if (A.face_hits || A.link) {
@@ -823,10 +836,27 @@ void k_generation(TraceArgs A) {
 }
 
 // ------------------------------------------------------------- variants
-static void launch_generation(uint32_t variant, dim3 grid, hipStream_t stream, const TraceArgs &A) {
-    if (variant == V_SPHERES) hipLaunchKernelGGL((k_generation<V_SPHERES>), grid, dim3(RPX_BLOCK), 0, stream, A);
-    else if (variant == V_LENS) hipLaunchKernelGGL((k_generation<V_LENS>), grid, dim3(RPX_BLOCK), 0, stream, A);
-    else hipLaunchKernelGGL((k_generation<V_ALL>), grid, dim3(RPX_BLOCK), 0, stream, A);
+// Rays per tile of a float64 chain.  Two 512-lane workgroups fill a CU at the
+// lens variants' four waves per SIMD, and their tiles halve the look-backs and
+// the staging: 4,194,304 rays of the asphere and doublet 0.54 -> 0.48 ms per
+// generation (1,024-ray tiles: 0.49 ms); a lens of eight surfaces, kernels per
+// trace, 256- against 512-ray tiles: 8,000 rays 114 / 124 us, 65,536 rays 156 /
+// 160, 100,000 rays 172 / 160, 200,000 rays 225 / 211.  V_ALL keeps 256: its three
+// waves per SIMD leave a 512-lane workgroup's second one no room (Michelson:
+// 25 % slower).
+static uint32_t gen_block(uint32_t variant, uint64_t n_in) {
+    return variant != V_ALL && n_in >= 65536 ? 512u : 256u;
+}
+
+template <int B>
+static void launch_generation_b(uint32_t variant, dim3 grid, hipStream_t stream, const TraceArgs &A) {
+    if (variant == V_SPHERES) hipLaunchKernelGGL((k_generation<V_SPHERES, B>), grid, dim3(B), 0, stream, A);
+    else hipLaunchKernelGGL((k_generation<V_LENS, B>), grid, dim3(B), 0, stream, A);
+}
+static void launch_generation(uint32_t variant, uint32_t block, dim3 grid, hipStream_t stream, const TraceArgs &A) {
+    if (variant == V_ALL) hipLaunchKernelGGL((k_generation<V_ALL, 256>), grid, dim3(256), 0, stream, A);
+    else if (block == 512) launch_generation_b<512>(variant, grid, stream, A);
+    else launch_generation_b<256>(variant, grid, stream, A);
 }
 
 static void launch_gausslet_generation(uint32_t variant, dim3 grid, hipStream_t stream, const TraceArgs &A) {
@@ -966,7 +996,7 @@ static rpx_status_t run_generation(const rpx_scene_t *scene, int one_list, int o
                            A.ws.ctl);
         HIP_TRY(hipGetLastError());
         if (timing) HIP_TRY(hipEventRecord(ev.e[1], stream));
-        launch_generation(variant, dim3((unsigned)nb), stream, A);
+        launch_generation(variant, RPX_BLOCK, dim3((unsigned)nb), stream, A);
         HIP_TRY(hipGetLastError());
         if (timing) HIP_TRY(hipEventRecord(ev.e[2], stream));
         GenControl ctl;
@@ -1113,6 +1143,7 @@ static rpx_status_t trace_rays_impl(const rpx_scene_t *scene, const rpx_rays_t *
     spec.count_last = count_last;
     if (rpx_status_t st = check_chain(spec, scene, workspace, workspace_bytes)) return st;
     const uint32_t variant = scene_variant(scene);
+    spec.block = gen_block(variant, n_in);
     TraceArgs A;
     A.S = scene->view;
     A.out = *pool;
@@ -1141,7 +1172,7 @@ static rpx_status_t trace_rays_impl(const rpx_scene_t *scene, const rpx_rays_t *
         A.tile_base = cg.tile_base;
         A.by_launch = cg.by_launch;
         A.lookback_ticks = cg.lookback_ticks;
-        launch_generation(variant, dim3((unsigned)grid), stream, A);
+        launch_generation(variant, spec.block, dim3((unsigned)grid), stream, A);
         return hipGetLastError();
     };
     return run_chain(spec, scene, workspace, launch, counts, offsets, n_traced, face_hits, (hipStream_t)stream_);
