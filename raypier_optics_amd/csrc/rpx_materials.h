@@ -593,12 +593,28 @@ RPX_DEV void eval_children(const rpx_material_t &m, const Ray &in, uint32_t idx,
     }
 }
 
+// Real indices inside and outside of a refracting material, for its parabasal
+// rays (once per gausslet: a dispersive material takes them from its curves).
+struct ParaIndex {
+    double inside, outside;
+};
+
+template <uint32_t F>
+RPX_DEV ParaIndex parabasal_index(const rpx_material_t &m, double wavelength) {
+    if constexpr ((F & M_COATED) != 0) {
+        if (m.type == RPX_MAT_COATED_DISPERSIVE)
+            return ParaIndex{eval_dispersion(m.disp_inside, wavelength).re, eval_dispersion(m.disp_outside, wavelength).re};
+    }
+    return ParaIndex{m.n_inside[0], m.n_outside[0]};
+}
+
 // eval_parabasal_ray_c: InterfaceMaterial default (ctracer.pyx:1588-1610),
 // DielectricMaterial (cmaterials.pyx:683-724, inherited by FullDielectric and
 // SingleLayerCoated), CoatedDispersiveMaterial (:1393-1434), grating (:1544-1599).
+// n_re: the base child's index, ray_type_id: its type.
 template <uint32_t F>
-RPX_DEV Para eval_parabasal(const rpx_material_t &m, const Ray &base, V3 direction, V3 point,
-                            const Orientation &orient, uint32_t ray_type_id, const WlTable &wavelengths) {
+RPX_DEV Para eval_parabasal(const rpx_material_t &m, const ParaIndex &index, double wavelength, double n_re,
+                            V3 direction, V3 point, const Orientation &orient, uint32_t ray_type_id) {
     Para out;
     V3 normal = unit(orient.normal);
     switch (m.type) {
@@ -610,41 +626,27 @@ RPX_DEV Para eval_parabasal(const rpx_material_t &m, const Ray &base, V3 directi
         direction = unit(direction);
         double cosTheta = dot(normal, direction);
         V3 ctn = mul(normal, cosTheta);
-        double n1, n2;
-        int flip;
-        double nin, nout;
-        if (m.type == RPX_MAT_COATED_DISPERSIVE) {
-            double wvl = wavelengths[base.wl_idx];
-            nin = eval_dispersion(m.disp_inside, wvl).re;
-            nout = eval_dispersion(m.disp_outside, wvl).re;
-        } else {
-            nin = m.n_inside[0];
-            nout = m.n_outside[0];
-        }
-        if (cosTheta < 0.0) { n1 = nout; n2 = nin; flip = 1; }
-        else { n1 = nin; n2 = nout; flip = -1; }
         if (ray_type_id & RPX_REFL_RAY) {
             out.direction = sub(direction, mul(ctn, 2));
         } else {
-            V3 tangent = sub(direction, ctn);
-            V3 tg2 = mul(tangent, n1 / n2);
-            double tan_mag_sq = mag_sq(tg2);
-            double c2 = sqrt(1 - tan_mag_sq);
-            out.direction = sub(tg2, mul(normal, c2 * flip));
+            const bool inward = cosTheta < 0.0;
+            const double n1 = inward ? index.outside : index.inside, n2 = inward ? index.inside : index.outside;
+            V3 tg2 = mul(sub(direction, ctn), n1 / n2);
+            double c2 = sqrt(1 - mag_sq(tg2));
+            out.direction = sub(tg2, mul(normal, inward ? c2 : -c2));
         }
     } break;
     case RPX_MAT_GRATING: {
         if constexpr ((F & M_GRATING) == 0) break;
         V3 tangent = unit(orient.tangent);
         V3 tangent2 = cross(normal, tangent);
-        double wavelen = wavelengths[base.wl_idx];
         double line_spacing = 1000.0 / m.lines_per_mm;
         V3 reflected = unit(direction);
         double k_z = dot(normal, reflected);
         double k_y = dot(tangent2, reflected);
         double k_x = dot(tangent, reflected);
         int sign = (k_z < 0.0) ? 1 : -1;
-        k_x = k_x - m.order * wavelen / (line_spacing * base.n.re);
+        k_x = k_x - m.order * wavelength / (line_spacing * n_re);
         k_z = 1 - (k_x * k_x) - (k_y * k_y);
         k_z = sign * sqrt(k_z);
         reflected = mul(tangent, k_x);

@@ -440,28 +440,6 @@ struct TraceArgs {
     uint64_t lookback_ticks = 0;
 };
 
-struct CountEmit {
-    static constexpr int kCap = 3;
-    int n = 0;
-    RPX_DEV void operator()(const Ray &) { ++n; }
-    RPX_DEV void skip() { ++n; }
-};
-
-// Writes at most `room` children (the count reserved by the counting pass),
-// so a lane can never write outside its slot range.
-struct StoreEmit {
-    static constexpr int kCap = 3;
-    const rpx_rays_t *out;
-    uint64_t pos;
-    uint32_t room;
-    RPX_DEV void operator()(const Ray &r) {
-        if (room == 0) return;
-        store_ray(*out, pos++, r);
-        --room;
-    }
-    RPX_DEV void skip() {}
-};
-
 // After a generation's children are placed: stores children from index 2 on
 // (a multi-order grating's third order) at pos + index, within `limit`.
 struct TailEmit {
@@ -476,16 +454,12 @@ struct TailEmit {
     RPX_DEV void skip() { ++n; }
 };
 
-// Collects up to 3 children of one gausslet base ray.
-struct CollectEmit {
+// Keeps the last child of one ray.
+struct LastEmit {
     static constexpr int kCap = 3;
-    Ray r[3];
-    int n = 0;
-    RPX_DEV void operator()(const Ray &x) {
-        if (n < 3) r[n] = x;
-        ++n;
-    }
-    RPX_DEV void skip() { ++n; }
+    Ray r;
+    RPX_DEV void operator()(const Ray &x) { r = x; }
+    RPX_DEV void skip() {}
 };
 
 // One gausslet generation in one launch (trace_gausslet_c, ctracer.pyx:
@@ -493,12 +467,20 @@ struct CollectEmit {
 // gausslet; the base ray's nearest-face search and its parabasal rays'
 // intersections with that face (every one must hit it, lengths updated in
 // place) come first, with the child count from the material; the decoupled
-// look-back then places the children, and the lane builds them and their
-// parabasal rays straight into their slots (children's lengths reset to
-// max_length, :2280).  Gausslet children are built after the look-back, not
-// held in registers through it: a child carries six parabasal rays.
+// look-back then places the children, whose base rays stay in registers
+// through it (children's lengths reset to max_length, :2280); the parabasal
+// rays of the children are built from the parents' after it, a child's six
+// being too many to hold.  Bound by memory latency: 262,144 gausslets are four
+// tiles per CU, one round of waves, so the next parabasal ray is loaded while
+// the current one is worked on, and the kernel stays at 128 registers (four
+// waves per SIMD; three for V_ALL, which needs 168).  MI355X, 262,144 gausslets
+// through a plano-convex lens: 175 -> 98 us and 136 -> 94 us for the two
+// generations with children, 20 -> 8 us for the last, against evaluating the
+// children twice, through scratch memory (a generation with children moves
+// 0.31 GB, 66 us at the 4.76 TB/s that a large copy reaches).
 template <uint32_t F>
-__global__ __launch_bounds__(RPX_BLOCK) void k_gausslet_generation(TraceArgs A) {
+__global__ __launch_bounds__(RPX_BLOCK) __attribute__((amdgpu_waves_per_eu(F == V_ALL ? 3 : 4)))
+void k_gausslet_generation(TraceArgs A) {
     __shared__ SceneLds lds_scene;
     __shared__ uint32_t lds_hist[RPX_LDS_FACES];
     __shared__ uint32_t lds_wave[RPX_BLOCK / 64];
@@ -524,6 +506,19 @@ __global__ __launch_bounds__(RPX_BLOCK) void k_gausslet_generation(TraceArgs A) 
         if (blockIdx.x >= n_tiles) return;
         if (threadIdx.x == 0) my_tile = atomicAdd(&A.ws.ctl->tile_counter, 1u);
     }
+    const double *f = in.f64;
+    const uint64_t c = in.capacity;
+    V3 origin = v3(0, 0, 0), dir = v3(0, 0, 0);
+    uint32_t wl_idx = 0;
+    auto load_geometry = [&](uint64_t i) {
+        origin = v3(f[RPX_OX * c + i], f[RPX_OY * c + i], f[RPX_OZ * c + i]);
+        dir = v3(f[RPX_DX * c + i], f[RPX_DY * c + i], f[RPX_DZ * c + i]);
+        wl_idx = in.u32[RPX_WL_IDX * c + i];
+    };
+    if (A.by_launch) {   // as k_generation: these loads overlap the staging
+        const uint64_t i0 = (uint64_t)my_tile * RPX_BLOCK + threadIdx.x;
+        if (i0 < n_in) load_geometry(i0);
+    }
     const SceneView S = stage_scene(A.S, lds_scene);
     if (threadIdx.x < RPX_LDS_FACES) lds_hist[threadIdx.x] = 0;
     if (threadIdx.x == 0) {
@@ -534,13 +529,21 @@ __global__ __launch_bounds__(RPX_BLOCK) void k_gausslet_generation(TraceArgs A) 
     __syncthreads();
     const uint32_t tile = lds_tile;
     const uint64_t i = (uint64_t)tile * RPX_BLOCK + threadIdx.x;
-    const uint64_t c = in.capacity;
-    uint32_t count = 0;
+    PairEmit ce;
+    WlOne wavelength{0.0};
     int hit_rec = -1, hit_list = -1;
+    // geometry and length of parabasal ray j
+    struct ParaIn {
+        V3 origin, direction;
+        double length;
+    };
+    auto load_para = [&](int j) {
+        const double *P = in.para + (uint64_t)j * RPX_PARA_FIELDS * c + i;
+        return ParaIn{v3(P[0], P[c], P[2 * c]), v3(P[3 * c], P[4 * c], P[5 * c]), P[9 * c]};
+    };
     if (i < n_in) {
-        const double *f = in.f64;
-        V3 origin = v3(f[RPX_OX * c + i], f[RPX_OY * c + i], f[RPX_OZ * c + i]);
-        V3 dir = v3(f[RPX_DX * c + i], f[RPX_DY * c + i], f[RPX_DZ * c + i]);
+        if (!A.by_launch) load_geometry(i);
+        wavelength.v = A.count_children ? A.wavelengths[wl_idx] : 0.0;
         // in a chain every gausslet starts at max_length (trace_rays resets
         // the input, children are written so), which keeps a generation
         // repeatable after a run-out look-back (its in-place lengths are then
@@ -548,115 +551,133 @@ __global__ __launch_bounds__(RPX_BLOCK) void k_gausslet_generation(TraceArgs A) 
         const NearHit nh = nearest_face<F, F != V_ALL>(S, A.S.faces, origin, dir, A.max_length,
                                                        A.link ? A.max_length : f[RPX_LENGTH * c + i], A.one_list,
                                                        A.one_face);
-        const double length = nh.length;
-        const uint32_t end_face = nh.end_face;
         hit_rec = nh.rec;
         hit_list = nh.list;
-        in.f64[RPX_LENGTH * c + i] = length;
-        in.u32[RPX_END_FACE_IDX * c + i] = end_face;
         if (hit_rec >= 0) {
             atomicAdd(&lds_hist[hit_rec], 1u);
             atomicAdd(&lds_hits, 1u);
             const rpx_face_t &fc = S.faces[hit_rec];
             const rpx_face_list_t &fl = S.face_lists[hit_list];
             // trace_parabasal_rays (ctracer.pyx:2363-2373): every parabasal
-            // ray must hit the same face; lengths update in place
+            // ray must hit the same face; lengths update in place.  The next
+            // ray is loaded before the current one is tested.
             bool para_ok = true;
-            const double *P = in.para;
+            ParaIn next = load_para(0);
             for (int j = 0; j < RPX_N_PARA && para_ok; ++j) {
-                const uint64_t b = (uint64_t)j * RPX_PARA_FIELDS;
-                V3 po = v3(P[(b + 0) * c + i], P[(b + 1) * c + i], P[(b + 2) * c + i]);
-                V3 pd = v3(P[(b + 3) * c + i], P[(b + 4) * c + i], P[(b + 5) * c + i]);
-                double plen = A.link ? A.max_length : P[(b + 9) * c + i];
-                V3 pend = add(po, mul(pd, A.max_length));
-                double dist = face_intersect<F>(S, fc, make_seg(to_local(fl, po), to_local(fl, pend)), 0);
-                if (fc.tolerance < dist && dist < plen) {
-                    in.para[(b + 9) * c + i] = dist;
+                const ParaIn p = next;
+                if (j + 1 < RPX_N_PARA) next = load_para(j + 1);
+                const V3 pend = add(p.origin, mul(p.direction, A.max_length));
+                const double dist = face_intersect<F>(S, fc, make_seg(to_local(fl, p.origin), to_local(fl, pend)), 0);
+                if (fc.tolerance < dist && dist < (A.link ? A.max_length : p.length)) {
+                    in.para[((uint64_t)j * RPX_PARA_FIELDS + 9) * c + i] = dist;
                 } else {
                     para_ok = false;
                 }
             }
             if (para_ok && A.count_children && fc.material >= 0) {
-                Ray r = load_ray(in, i);
-                r.length = length;
-                r.end_face_idx = end_face;
-                V3 hp = add(r.origin, mul(r.direction, length));
+                Ray r = load_ray_rest(in, i);
+                r.origin = origin;
+                r.direction = dir;
+                r.wl_idx = wl_idx;
+                r.length = nh.length;
+                r.end_face_idx = nh.end_face;
+                V3 hp = add(origin, mul(dir, nh.length));
                 Orientation o = compute_orientation<F>(S, fl, fc, hp);
-                CountEmit ce;
-                eval_children<F>(S.materials[fc.material], r, (uint32_t)i, hp, o, A.wavelengths, ce);
-                count = (uint32_t)min(ce.n, 3);
+                eval_children<F>(S.materials[fc.material], r, (uint32_t)i, hp, o, wavelength, ce);
             }
         }
+        in.f64[RPX_LENGTH * c + i] = nh.length;
+        in.u32[RPX_END_FACE_IDX * c + i] = nh.end_face;
     }
-    uint32_t block_total;
-    const uint32_t local = block_scan_small(count, lds_wave, &block_total);
-    {
-        const uint64_t mp = __ballot(count > 0);
-        if ((threadIdx.x & 63) == 0 && mp) atomicAdd(&lds_parents, (uint32_t)__popcll(mp));
-    }
-    if (threadIdx.x < 64) {
-        const uint64_t excl = lookback_tagged(A.ws.tile_status, tile, 0, block_total, &A.ws.ctl->error, A.status_tag,
-                                              A.lookback_ticks);
-        if (threadIdx.x == 0) lds_excl = excl;
-    }
-    __syncthreads();
-    const uint64_t pos = lds_excl + local;
-    if (count > 0 && pos + count <= out_limit) {
-        const rpx_face_t &fc = S.faces[hit_rec];
-        const rpx_face_list_t &fl = S.face_lists[hit_list];
-        const rpx_material_t &m = S.materials[fc.material];
-        Ray r = load_ray(in, i);
-        V3 hp = add(r.origin, mul(r.direction, r.length));
-        Orientation o = compute_orientation<F>(S, fl, fc, hp);
-        CollectEmit ce;
-        eval_children<F>(m, r, (uint32_t)i, hp, o, A.wavelengths, ce);
-        const uint64_t co = out.capacity;
-        const int nk = min(min(ce.n, 3), (int)count);
-        for (int k = 0; k < nk; ++k) {
-            Ray child = ce.r[k];
-            child.length = A.max_length;
-            store_ray(out, pos + k, child);
+    const uint32_t count = (uint32_t)min(ce.n, 3);
+    if (A.count_children) {
+        uint32_t block_total;
+        const uint32_t local = block_scan_small(count, lds_wave, &block_total);
+        {
+            const uint64_t mp = __ballot(count > 0);
+            if ((threadIdx.x & 63) == 0 && mp) atomicAdd(&lds_parents, (uint32_t)__popcll(mp));
         }
-        for (int j = 0; j < RPX_N_PARA; ++j) {
-            const uint64_t b = (uint64_t)j * RPX_PARA_FIELDS;
-            const double *P = in.para;
-            V3 po = v3(P[(b + 0) * c + i], P[(b + 1) * c + i], P[(b + 2) * c + i]);
-            V3 pd = v3(P[(b + 3) * c + i], P[(b + 4) * c + i], P[(b + 5) * c + i]);
-            double plen = P[(b + 9) * c + i];
-            V3 pp = add(po, mul(pd, plen));
-            Orientation po_ = compute_orientation<F>(S, fl, fc, pp);
-            for (int k = 0; k < nk; ++k) {
-                Para q = eval_parabasal<F>(m, ce.r[k], pd, pp, po_, ce.r[k].ray_type_id, A.wavelengths);
-                double *Q = out.para;
-                const uint64_t oi = pos + k;
-                Q[(b + 0) * co + oi] = q.origin.x;
-                Q[(b + 1) * co + oi] = q.origin.y;
-                Q[(b + 2) * co + oi] = q.origin.z;
-                Q[(b + 3) * co + oi] = q.direction.x;
-                Q[(b + 4) * co + oi] = q.direction.y;
-                Q[(b + 5) * co + oi] = q.direction.z;
-                Q[(b + 6) * co + oi] = q.normal.x;
-                Q[(b + 7) * co + oi] = q.normal.y;
-                Q[(b + 8) * co + oi] = q.normal.z;
-                Q[(b + 9) * co + oi] = A.max_length;
+        if (threadIdx.x < 64) {
+            const uint64_t excl = lookback_tagged(A.ws.tile_status, tile, 0, block_total, &A.ws.ctl->error,
+                                                  A.status_tag, A.lookback_ticks);
+            if (threadIdx.x == 0) lds_excl = excl;
+        }
+        __syncthreads();
+        const uint64_t pos = lds_excl + local;
+        if (count > 0 && pos + count <= out_limit) {
+            const rpx_face_t &fc = S.faces[hit_rec];
+            const rpx_face_list_t &fl = S.face_lists[hit_list];
+            const rpx_material_t &m = S.materials[fc.material];
+            const uint64_t co = out.capacity;
+            ParaIn next = load_para(0);
+            ce.length = A.max_length;
+            store_ray(out, pos, ce.first());
+            if (count > 1) store_ray(out, pos + 1, ce.second());
+            // what the parabasal rays take from the children: their kind, and the
+            // index the ray travelled in (gratings)
+            const uint32_t type0 = count > 1 ? ce.s1.type : ce.s0.type, type1 = ce.s0.type;
+            const double n0 = count > 1 ? ce.s1.n.re : ce.s0.n.re, n1 = ce.s0.n.re;
+            const ParaIndex index = parabasal_index<F>(m, wavelength.v);
+            auto store_para = [&](int j, uint64_t slot, const ParaIn &p, V3 pp, const Orientation &po, double n_re,
+                                  uint32_t type) {
+                const Para q = eval_parabasal<F>(m, index, wavelength.v, n_re, p.direction, pp, po, type);
+                double *Q = out.para + (uint64_t)j * RPX_PARA_FIELDS * co + slot;
+                Q[0] = q.origin.x;
+                Q[co] = q.origin.y;
+                Q[2 * co] = q.origin.z;
+                Q[3 * co] = q.direction.x;
+                Q[4 * co] = q.direction.y;
+                Q[5 * co] = q.direction.z;
+                Q[6 * co] = q.normal.x;
+                Q[7 * co] = q.normal.y;
+                Q[8 * co] = q.normal.z;
+                Q[9 * co] = A.max_length;
+            };
+            for (int j = 0; j < RPX_N_PARA; ++j) {
+                const ParaIn p = next;
+                if (j + 1 < RPX_N_PARA) next = load_para(j + 1);
+                const V3 pp = add(p.origin, mul(p.direction, p.length));
+                const Orientation po = compute_orientation<F>(S, fl, fc, pp);
+                for (uint32_t k = 0; k < min(count, 2u); ++k)
+                    store_para(j, pos + k, p, pp, po, k == 0 ? n0 : n1, k == 0 ? type0 : type1);
+            }
+            if constexpr ((F & M_GRATING) != 0) {
+                if (count > 2) {
+                    // a grating's third order is built again, as in k_generation
+                    Ray r = load_ray(in, i);
+                    const V3 hp = add(r.origin, mul(r.direction, r.length));
+                    const Orientation o = compute_orientation<F>(S, fl, fc, hp);
+                    LastEmit last;
+                    eval_children<F>(m, r, (uint32_t)i, hp, o, wavelength, last);
+                    last.r.length = A.max_length;
+                    store_ray(out, pos + 2, last.r);
+                    for (int j = 0; j < RPX_N_PARA; ++j) {
+                        const ParaIn p = load_para(j);
+                        const V3 pp = add(p.origin, mul(p.direction, p.length));
+                        const Orientation po = compute_orientation<F>(S, fl, fc, pp);
+                        store_para(j, pos + 2, p, pp, po, last.r.n.re, last.r.ray_type_id);
+                    }
+                }
             }
         }
-    }
-    if (threadIdx.x == 0) {
-        add_hits(A.ws.ctl, tile, lds_hits);
-        if (lds_parents) atomicAdd(&A.ws.ctl->parent_shards[tile % RPX_SHARDS], lds_parents);
-        if ((uint64_t)tile == (n_in - 1) / RPX_BLOCK) {
-            const uint64_t kids = lds_excl + block_total;
-            A.ws.ctl->children = kids;
-            if (A.link) {
-                const uint64_t at = A.link[0].out_offset;
-                A.link[1].count = kids;
-                A.link[1].offset = at;
-                A.link[1].out_offset = at + kids;
-                A.head_out->children = kids;   // host-mapped: read once the generation has ended
+        if (threadIdx.x == 0) {
+            if (lds_parents) atomicAdd(&A.ws.ctl->parent_shards[tile % RPX_SHARDS], lds_parents);
+            if ((uint64_t)tile == (n_in - 1) / RPX_BLOCK) {
+                const uint64_t kids = lds_excl + block_total;
+                A.ws.ctl->children = kids;
+                if (A.link) {
+                    const uint64_t at = A.link[0].out_offset;
+                    A.link[1].count = kids;
+                    A.link[1].offset = at;
+                    A.link[1].out_offset = at + kids;
+                    A.head_out->children = kids;   // host-mapped: read once the generation has ended
+                }
             }
         }
+    } else {
+        __syncthreads();   // lds_hist and lds_hits are complete
     }
+    if (threadIdx.x == 0) add_hits(A.ws.ctl, tile, lds_hits);
     uint32_t *shard = A.ws.ctl->face_shards[tile % RPX_SHARDS];
     for (int k = threadIdx.x; k < S.n_list_faces; k += blockDim.x) {
         uint32_t h = lds_hist[k];
@@ -777,8 +798,8 @@ void k_generation(TraceArgs A) {
             if ((threadIdx.x & 63) == 0) atomicAdd(&lds_hits, (uint32_t)__popcll(mh));
         }
         if (threadIdx.x < 64) {
-            const uint64_t excl = lookback_tagged(A.ws.tile_status, tile, 0, block_total, &A.ws.ctl->error, A.status_tag,
-                                                  A.lookback_ticks);
+            const uint64_t excl = lookback_tagged(A.ws.tile_status, tile, 0, block_total, &A.ws.ctl->error,
+                                                  A.status_tag, A.lookback_ticks);
             if (threadIdx.x == 0) lds_excl = excl;
         }
         __syncthreads();
