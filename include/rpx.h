@@ -818,7 +818,7 @@ rpx_status_t rpx_lens_eval(const rpx_lens_t *lens, const double *zcart, const rp
  * grad[s*6 + q] = d(objective)/d(param[s][q]);
  * grad[6*n_surfaces + s*RPX_LENS_ZTERMS + k] = d(objective)/d(C[s][k]) (0
  * where the surface has no distortion), given the moments of rpx_lens_eval
- * for the same inputs.  Intersections are recomputed, not stored. */
+ * for the same inputs.  Rays are traced again, nothing is kept between calls. */
 rpx_status_t rpx_lens_grad(const rpx_lens_t *lens, const double *zcart, const rpx_rays_t *rays, uint64_t n_rays,
                            const double *n_table, uint64_t n_wavelengths, int32_t objective, const double *moments,
                            double *grad, void *workspace, uint64_t workspace_bytes, void *stream);

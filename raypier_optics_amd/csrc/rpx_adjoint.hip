@@ -4,20 +4,19 @@
 //
 // Forward (k_lens_forward): one thread per ray traces surfaces 0..n-1 and the
 // detector plane and writes per-workgroup moment partials.  Adjoint
-// (k_lens_adjoint): each thread traces its ray again, keeping the state
-// entering every surface (direction and distance; the points follow from
-// the last one), then runs the chain rule backwards from the detector, recomputing
-// each surface's normal and refraction; surface parameters receive the
-// contributions of the implicit intersection equation and of the normal.
+// (k_lens_adjoint): each thread traces its ray again, keeping the direction
+// entering every surface and the distance to it (the points follow from the
+// last one), then runs the chain rule backwards from the detector,
+// recomputing each surface's normal and refraction; surface parameters receive
+// the contributions of the implicit intersection equation and of the normal.
 // Per-workgroup parameter partials are summed by a fixed-order reduction.
 //
 // Both are bound by float64 instruction issue (the rays are 56 bytes each).  A
 // surface's w and 1/w come from one reciprocal root, 1/(1+w) and every other
 // quotient from reciprocals, and products are fused with the sums that take
-// them.
-// The adjoint also moves the kept states through private memory:
-// 32 bytes per surface (with the 48 of point and direction it takes 309 us at
-// the size below, not 251).  MI355X, 2,097,152 rays through 8 surfaces: forward
+// them.  The adjoint also moves the kept states through private memory: 32
+// bytes per surface (with the 48 of point and direction it takes 309 us at the
+// size below, not 251).  MI355X, 2,097,152 rays through 8 surfaces: forward
 // 313 -> 124 us, adjoint 777 -> 251 us (3 waves per SIMD instead of 5: 283 us),
 // column sums 14 -> 10 us, against square roots and divisions per term, two
 // Newton steps more, and every intersection solved twice.
@@ -447,7 +446,8 @@ __device__ __forceinline__ void lens_adjoint(const LensArgs &A, const double *mo
             //   dS/dk = c^3 rho^2 y v^2 / 2,      dS'/dk = c^3 rho y^3 / 4
             const double c = P[0], u = (1 + P[1]) * c * c, y3 = k.y * k.y * k.y, v = rcp_third(k.w1);
             const double yv2 = k.y * v * v, r2 = rho * rho, r3 = r2 * rho, c3 = c * c * c;
-            const double rhob = Spb * (0.25 * c * u * y3 + 2 * P[2] + rho * (6 * P[3] + rho * (12 * P[4] + rho * (20 * P[5]))));
+            const double rhob =
+                Spb * (0.25 * c * u * y3 + 2 * P[2] + rho * (6 * P[3] + rho * (12 * P[4] + rho * (20 * P[5]))));
             qb.x += 2 * q.x * rhob;
             qb.y += 2 * q.y * rhob;
             // intersection q = p + t d with G(t; p, d, param) = 0; the
