@@ -16,7 +16,7 @@
 // quotient from reciprocals, and products are fused with the sums that take
 // them.  The adjoint also moves the kept states through private memory: 32
 // bytes per surface (with the 48 of point and direction it takes 309 us at the
-// size below, not 251).  MI355X, 2,097,152 rays through 8 surfaces: forward
+// size below, not 251).  MI355X, 2,097,152 rays through 6 surfaces: forward
 // 313 -> 124 us, adjoint 777 -> 251 us (3 waves per SIMD instead of 5: 283 us),
 // column sums 14 -> 10 us, against square roots and divisions per term, two
 // Newton steps more, and every intersection solved twice.

@@ -860,7 +860,7 @@ void k_generation(TraceArgs A) {
 // Rays per tile of a float64 chain.  Two 512-lane workgroups fill a CU at the
 // lens variants' four waves per SIMD, and their tiles halve the look-backs and
 // the staging: 4,194,304 rays of the asphere and doublet 0.54 -> 0.48 ms per
-// generation (1,024-ray tiles: 0.49 ms); a lens of eight surfaces, kernels per
+// generation (1,024-ray tiles: 0.49 ms); a lens of six surfaces, kernels per
 // trace, 256- against 512-ray tiles: 8,000 rays 114 / 124 us, 65,536 rays 156 /
 // 160, 100,000 rays 172 / 160, 200,000 rays 225 / 211.  V_ALL keeps 256: its three
 // waves per SIMD leave a 512-lane workgroup's second one no room (Michelson:
