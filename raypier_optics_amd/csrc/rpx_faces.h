@@ -253,8 +253,9 @@ RPX_DEV V3 to_global_dir(const rpx_face_list_t &fl, V3 d) {
 }
 
 // ----------------------------------------------------------- conic / asphere
-// intersect_conic (cfaces.pyx:1695-1747) for a unit direction d: the distance.
-RPX_DEV double intersect_conic(V3 a, V3 d, double curvature, double conic_const) {
+// intersect_conic (cfaces.pyx:1695-1747) for a unit direction d: the distance
+// t, or false where the ray misses the conic.
+RPX_DEV bool intersect_conic(V3 a, V3 d, double curvature, double conic_const, double &t) {
     const double beta = 1 + conic_const;
     const double R = -curvature;
     const double b2 = beta * beta;
@@ -264,9 +265,10 @@ RPX_DEV double intersect_conic(V3 a, V3 d, double curvature, double conic_const)
     const double B = fma(beta, fma(-R, d.z, ad), b2 * (a.z * d.z));
     const double C = fma(beta, fma(-2 * R, a.z, at), b2 * (a.z * a.z));
     double D = fma(B, B, -(A * C));
-    if (D < 0) return -1;
+    if (D < 0) return false;
     D = sqrt(D);
-    return (R * beta * d.z <= 0 ? -B + D : -B - D) / A;
+    t = (R * beta * d.z <= 0 ? -B + D : -B - D) / A;
+    return true;
 }
 
 // x = r^2 polynomial A4 x^2 + .. + A16 x^8 and its derivative, by Horner's rule
@@ -435,7 +437,8 @@ RPX_DEV double plain_intersect(const SceneView &S, const rpx_face_t &f, const Se
         if constexpr ((F & F_CONIC) == 0) return -1;  // cfaces.pyx:1767-1798
         V3 a = g.p1;
         a.z -= f.p[1];
-        const double t = intersect_conic(a, g.u, f.p[0], f.p[2]);
+        double t;
+        if (!intersect_conic(a, g.u, f.p[0], f.p[2], t)) return -1;
         if (is_base && !shape_inside(S, f.shape, fma(g.u.x, t, a.x), fma(g.u.y, t, a.y))) return -1;
         return in_segment(g, t, tol) ? t : -1;
     }
@@ -446,13 +449,16 @@ RPX_DEV double plain_intersect(const SceneView &S, const rpx_face_t &f, const Se
         // (a.z + t u.z), w = sqrt(1 - beta r^2 / R^2); the conic term's
         // derivative in r^2 is 1 / (2 R w) (the reference's two fractions,
         // cfaces.pyx:1866-1882, added up), so a step takes one square root and
-        // one division.
+        // one division.  A ray that misses the conic starts at h = -1 as in the
+        // reference, a whole segment behind p1: from nearer by, the iteration
+        // finds roots that the reference does not accept.
         const double atol = f.p[10] * g.slen;
         const double tl = atol * atol;
         V3 a = g.p1;
         a.z -= f.p[1];
         const double R = -f.p[0], k2 = (1 + f.p[2]) / (R * R);
-        double t = intersect_conic(a, g.u, f.p[0], f.p[2]);
+        double t;
+        if (!intersect_conic(a, g.u, f.p[0], f.p[2], t)) t = -g.slen;
         double f_last = RPX_INF, dt = RPX_INF;
         bool converged = false;
         for (int i = 0; i <= 100; ++i) {
