@@ -5,21 +5,24 @@
 // Forward (k_lens_forward): one thread per ray traces surfaces 0..n-1 and the
 // detector plane and writes per-workgroup moment partials.  Adjoint
 // (k_lens_adjoint): each thread traces its ray again, keeping the direction
-// entering every surface and the distance to it (the points follow from the
-// last one), then runs the chain rule backwards from the detector,
-// recomputing each surface's normal and refraction; surface parameters receive
-// the contributions of the implicit intersection equation and of the normal.
+// entering every surface, the distance to it and x and y there, then runs the
+// chain rule backwards from the detector, recomputing each surface's normal
+// and refraction at the very point; surface parameters receive the
+// contributions of the implicit intersection equation and of the normal.
 // Per-workgroup parameter partials are summed by a fixed-order reduction.
 //
 // Both are bound by float64 instruction issue (the rays are 56 bytes each).  A
 // surface's w and 1/w come from one reciprocal root, 1/(1+w) and every other
 // quotient from reciprocals, and products are fused with the sums that take
-// them.  The adjoint also moves the kept states through private memory: 32
-// bytes per surface (with the 48 of point and direction it takes 309 us at the
-// size below, not 251).  MI355X, 2,097,152 rays through 6 surfaces: forward
-// 313 -> 124 us, adjoint 777 -> 251 us (3 waves per SIMD instead of 5: 283 us),
-// column sums 14 -> 10 us, against square roots and divisions per term, two
-// Newton steps more, and every intersection solved twice.
+// them.  The adjoint also moves the kept states through private memory: 48
+// bytes per surface.  (32, with the points stepped back to from the last one,
+// take 261 us at the size below, not 281; but a point is then a rounding of the
+// segment away from the forward's, which near total reflection is all there is
+// of the refracted cosine.)  MI355X, 2,097,152 rays through 6 surfaces:
+// forward 315 -> 128 us, adjoint 774 -> 281 us (3 waves per SIMD instead of 5
+// cost another 32 us), column sums 15 -> 11 us, against square roots and
+// divisions per term, two Newton steps more, and every intersection solved
+// twice.
 //
 // Surface:  G(q) = S(rho) + D(q.x, q.y) - (q.z - z_s) = 0,
 //   rho     = q.x^2 + q.y^2,
@@ -57,9 +60,16 @@ struct Conic {
     double w, y, w1;    // w1 = 1 + w
 };
 
+// With TRACED (the backward pass, at a point where the forward pass had a root)
+// it has one always: the two passes may evaluate the same point to a rounding
+// of the argument's terms apart, and a ray of a surface's rim then keeps the
+// least argument that such a rounding leaves, instead of none.
+#define LEAST_ARG 0x1p-53
+template <bool TRACED>
 __device__ __forceinline__ bool conic(const double *P, double rho, Conic &k) {
-    const double arg = 1 - (1 + P[1]) * P[0] * P[0] * rho;
-    if (!(arg > 0)) return false;
+    double arg = 1 - (1 + P[1]) * P[0] * P[0] * rho;
+    if constexpr (TRACED) arg = fmax(arg, LEAST_ARG);
+    else if (!(arg > 0)) return false;
     k.y = rsq_third(arg);
     k.w = arg * k.y;
     k.w1 = 1 + k.w;
@@ -138,7 +148,7 @@ __device__ __forceinline__ bool newton_step(const double *P, const double *C, do
     const double qx = p.x + t * d.x, qy = p.y + t * d.y;
     const double rho = qx * qx + qy * qy;
     Conic k;
-    if (!conic(P, rho, k)) return false;
+    if (!conic<false>(P, rho, k)) return false;
     z = zernike_eval(C, Ru, qx, qy, false);
     Sp = slope(P, rho, k.y);
     const double G = P[0] * rho + k.w1 * (poly(P, rho) + z.D - (hz + t * d.z));     // (1 + w) G
@@ -172,15 +182,19 @@ struct Refr {
     V3 t;
 };
 
-__device__ __forceinline__ bool refract(V3 q, double Sp, const ZEval &z, V3 d, double mu, Refr &r) {
-    const V3 m = v3(-(2 * q.x * Sp + z.Dx), -(2 * q.y * Sp + z.Dy), 1.0);
+// TRACED as in conic: such a ray is not totally reflected.
+template <bool TRACED>
+__device__ __forceinline__ bool refract(double x, double y, double Sp, const ZEval &z, V3 d, double mu,
+                                        Refr &r) {
+    const V3 m = v3(-(2 * x * Sp + z.Dx), -(2 * y * Sp + z.Dy), 1.0);
     r.imlen = rsq_third(m.x * m.x + m.y * m.y + 1.0);
     const double c = (m.x * d.x + m.y * d.y + d.z) * r.imlen;
     r.sgn = c >= 0 ? 1.0 : -1.0;
     r.N = mul(m, r.imlen * r.sgn);
     r.cosv = c * r.sgn;
-    const double rr = 1 - mu * mu * (1 - r.cosv * r.cosv);
-    if (rr < 0) return false;
+    double rr = 1 - mu * mu * (1 - r.cosv * r.cosv);
+    if constexpr (TRACED) rr = fmax(rr, LEAST_ARG);
+    else if (rr < 0) return false;
     r.isr = rr > 0 ? rsq_third(rr) : RPX_INF;
     r.kappa = (rr > 0 ? rr * r.isr : rr) - mu * r.cosv;
     r.t = v3(mu * d.x + r.N.x * r.kappa, mu * d.y + r.N.y * r.kappa, mu * d.z + r.N.z * r.kappa);
@@ -197,12 +211,17 @@ struct LensArgs {
     int objective;
 };
 
+// Where a ray met a surface, and how far it came.
+struct Kept {
+    double x, y, t;
+};
+
 // Traces one ray: detector point (px, py), its wavefront path W and
-// wavelength index; when `keep`, the direction entering and the distance to
-// every surface, and the point on the last one.
+// wavelength index; when `keep`, the direction entering every surface and its
+// Kept, and the point on the last one.
 template <bool ZK, bool WF>
 __device__ __forceinline__ bool trace_ray(const LensArgs &A, uint64_t i, double &px, double &py, double &W,
-                                          uint32_t &wl, V3 &last, V3 *sd, double *st, bool keep) {
+                                          uint32_t &wl, V3 &last, V3 *sd, Kept *sq, bool keep) {
     const double *f = A.rays.f64;
     const uint64_t cap = A.rays.capacity;
     V3 p = v3(f[RPX_OX * cap + i], f[RPX_OY * cap + i], f[RPX_OZ * cap + i]);
@@ -221,9 +240,9 @@ __device__ __forceinline__ bool trace_ray(const LensArgs &A, uint64_t i, double 
                        q, t, Sp, z))
             return false;
         Refr r;
-        if (!refract(q, Sp, z, d, nt[A.L.medium_before[s]] / nt[A.L.medium_after[s]], r)) return false;
+        if (!refract<false>(q.x, q.y, Sp, z, d, nt[A.L.medium_before[s]] / nt[A.L.medium_after[s]], r)) return false;
         if constexpr (WF) W += nt[A.L.medium_before[s]] * t;
-        if (keep) st[s] = t;
+        if (keep) sq[s] = Kept{q.x, q.y, t};
         p = q;
         d = r.t;
     }
@@ -372,18 +391,18 @@ __device__ __forceinline__ void lens_adjoint(const LensArgs &A, const double *mo
     const uint64_t i = (uint64_t)blockIdx.x * LB + threadIdx.x;
     const double cnt = moments[0];
     const double obj = cnt > 0 ? objective_value(WF ? RPX_LENS_WAVEFRONT_RMS : RPX_LENS_SPOT_RMS, moments) : 0.0;
-    V3 q = v3(0, 0, 0), sd[RPX_LENS_MAX_SURFACES + 1];
-    double st[RPX_LENS_MAX_SURFACES];
+    V3 last = v3(0, 0, 0), sd[RPX_LENS_MAX_SURFACES + 1];
+    Kept sq[RPX_LENS_MAX_SURFACES];
     double px = 0, py = 0, W = 0;
     uint32_t wl = 0;
-    bool ok = (i < A.n) && cnt > 0 && obj > 0 && trace_ray<ZK, WF>(A, i, px, py, W, wl, q, sd, st, true);
+    bool ok = (i < A.n) && cnt > 0 && obj > 0 && trace_ray<ZK, WF>(A, i, px, py, W, wl, last, sd, sq, true);
     const double *nt = ok ? A.n_table + (uint64_t)wl * A.L.n_media : A.n_table;
     // seeds: adjoints of (p, d) leaving the last surface, and the weight of
     // each segment's optical path (wavefront objective)
     V3 pb = v3(0, 0, 0), db = v3(0, 0, 0);
     double omega = 0;
     if (ok) {
-        const V3 p = q, d = sd[S];
+        const V3 p = last, d = sd[S];
         if constexpr (!WF) {
             // d sigma / d (px, py) = (p - centroid) / (N sigma)
             const double cx = moments[1] / cnt, cy = moments[2] / cnt;
@@ -414,15 +433,15 @@ __device__ __forceinline__ void lens_adjoint(const LensArgs &A, const double *mo
         if (ok) {
             const double *P = A.L.param[s];
             const V3 d = sd[s];
-            const double t = st[s];
-            const double rho = q.x * q.x + q.y * q.y;
+            const Kept q = sq[s];
+            const double t = q.t, rho = q.x * q.x + q.y * q.y;
             Conic k;
-            conic(P, rho, k);      // traced: has a root
+            conic<true>(P, rho, k);
             const double Sp = slope(P, rho, k.y);
             const ZEval z = zernike_eval(C, Ru, q.x, q.y, true);
             const double mu = nt[A.L.medium_before[s]] / nt[A.L.medium_after[s]];
             Refr r;
-            refract(q, Sp, z, d, mu, r);
+            refract<true>(q.x, q.y, Sp, z, d, mu, r);
             // outputs of the step: q (adjoint pb), r.t (adjoint db)
             const V3 tb = db;
             V3 qb = pb;
@@ -489,7 +508,6 @@ __device__ __forceinline__ void lens_adjoint(const LensArgs &A, const double *mo
             }
             pb = pbar;
             db = dbar;
-            q = sub(q, mul(d, t));   // the point entering the surface
         }
         put4(&gsum[wave][s * 6], lane, wave_sum4(th[0], th[1], th[2], th[3]));
         put2(&gsum[wave][s * 6 + 4], lane, wave_sum2(th[4], th[5]));
