@@ -7,6 +7,7 @@ import ctypes
 
 from . import _abi
 from ._lib import load, check, require_gpu, stream_handle
+from .cmaterials import one_scan
 from .ctracer import RayCollection, GaussletCollection, _TraceContext, _generation, _wavelength_table
 
 
@@ -15,12 +16,13 @@ def _prepare(input_rays, face_lists, max_length, reset=True):
         input_rays.reset_length(max_length)
     wavelengths = numpy.asarray(input_rays.wavelengths)
     all_faces = list(chain(*(fs.faces for fs in face_lists)))
-    for i, f in enumerate(all_faces):
-        f.idx = i
-        f.count = 0
-        f.update()
-        f.material.wavelengths = wavelengths
-        f.max_length = max_length
+    with one_scan(wavelengths):
+        for i, f in enumerate(all_faces):
+            f.idx = i
+            f.count = 0
+            f.update()
+            f.material.wavelengths = wavelengths
+            f.max_length = max_length
     return all_faces
 
 

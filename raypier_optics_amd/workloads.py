@@ -27,7 +27,7 @@ from ._abi import ray_dtype, NO_FACE
 from .ctracer import RayCollection, FaceList
 from .cfaces import SphericalFace, CircularFace, AsphericFace, ShapedPlanarFace
 from .cshapes import CircleShape
-from .cmaterials import (BaseDispersionCurve, NondispersiveCurve, FullDielectricDispersiveMaterial,
+from .cmaterials import (one_scan, BaseDispersionCurve, NondispersiveCurve, FullDielectricDispersiveMaterial,
                          CoatedDispersiveMaterial, OpaqueMaterial)
 
 # Sellmeier formula-2 coefficients [0, B1, C1, B2, C2, B3, C3] (C in um^2)
@@ -142,11 +142,13 @@ def prepare_faces(face_lists, wavelengths, max_length):
     """Global face indices, counts and material wavelengths exactly as
     trace_rays sets them (core/tracer.py:28-34); returns all_faces."""
     all_faces = [f for fl in face_lists for f in fl.faces]
-    for i, f in enumerate(all_faces):
-        f.idx = i
-        f.count = 0
-        f.material.wavelengths = np.asarray(wavelengths)
-        f.max_length = max_length
+    wavelengths = np.asarray(wavelengths)
+    with one_scan(wavelengths):
+        for i, f in enumerate(all_faces):
+            f.idx = i
+            f.count = 0
+            f.material.wavelengths = wavelengths
+            f.max_length = max_length
     return all_faces
 
 
