@@ -22,7 +22,7 @@ _SLOT = 8 << 20
 def _slots(torch):
     """Two pinned slots (from torch's host allocator, which takes them back
     when the copies that use them have ended) and an event for each."""
-    return ([torch.empty(_SLOT, dtype=torch.uint8, pin_memory=True) for _ in range(2)],
+    return ([torch.empty(_SLOT, dtype=torch.uint8, device="cpu", pin_memory=True) for _ in range(2)],
             [torch.cuda.Event() for _ in range(2)])
 
 

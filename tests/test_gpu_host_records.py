@@ -42,3 +42,12 @@ def test_read_only_and_strided_records(gpu, n):
     b.flags.writeable = False
     d.upload(b)
     assert d.download(n).tobytes() == b.tobytes()
+
+
+def test_records_with_a_default_device(gpu):
+    """The pinned slots are host memory whatever torch's default device is."""
+    a = _records(20000, _abi.ray_dtype)     # 3.8 MB
+    d = DeviceRays(len(a))
+    with gpu.device("cuda"):
+        d.upload(a)
+        assert d.download(len(a)).tobytes() == a.tobytes()
