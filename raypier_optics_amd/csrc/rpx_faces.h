@@ -467,7 +467,9 @@ RPX_DEV double plain_intersect(const SceneView &S, const rpx_face_t &f, const Se
             const double w = sqrt(fma(-k2, r2, 1.0)), w1 = 1 + w;
             const double inv = 1.0 / (R * w * w1);
             const double fv = fma(r2 * w, inv, asph_poly(f, r2)) - fma(t, g.u.z, a.z);
-            if (i > 0 && fabs(fv) > fabs(f_last)) return -1;
+            // growing, or no number (outside the conic's domain), which no later
+            // step can mend: the reference runs its 100 steps on it
+            if (!(fabs(fv) <= fabs(f_last))) return -1;
             f_last = fv;
             const double slope = fma(w1, inv, 2 * asph_dpoly(f, r2));
             dt = -fv / fma(fma(g.u.x, tx, g.u.y * ty), slope, -g.u.z);
