@@ -252,6 +252,13 @@ RPX_DEV bool material_emits(const rpx_material_t &m) {
     return m.type != RPX_MAT_NONE && m.type != RPX_MAT_OPAQUE;
 }
 
+// power / P_in > threshold as a product: no reciprocal, which overflows for
+// the subnormal P_in of very faint rays.
+template <class T>
+RPX_DEV bool passes(T power, T P_in, T threshold) {
+    return P_in > 0 ? power > threshold * P_in : power < threshold * P_in;
+}
+
 // |a|^2
 RPX_DEV double cnorm2(Cx a) { return fma(a.re, a.re, a.im * a.im); }
 
@@ -541,7 +548,6 @@ RPX_DEV void eval_children(const rpx_material_t &m, const Ray &in, uint32_t idx,
         const Cx n1 = inward ? sd.n_out : sd.n_in, n3 = inward ? sd.n_in : sd.n_out;
         const double P_in = n1.re * (cnorm2(E1) + cnorm2(E2));
         if (P_in == 0.0) return;
-        const double per_P = 1.0 / P_in;
         // the tangential part of the direction, before and after refraction
         const V3 tangent = sub(in_dir, mul(normal, cosTheta));
         const V3 tg2 = mul(tangent, n1.re / n3.re);
@@ -566,7 +572,7 @@ RPX_DEV void eval_children(const rpx_material_t &m, const Ray &in, uint32_t idx,
                 return;
         }
         const Cx R_s = cmul(k.rs, E1), R_p = cmul(k.rp, E2);
-        if (n1.re * (cnorm2(R_s) + cnorm2(R_p)) * per_P > m.reflection_threshold) {
+        if (passes(n1.re * (cnorm2(R_s) + cnorm2(R_p)), P_in, m.reflection_threshold)) {
             sp.direction = sub(in_dir, mul(mul(normal, cosTheta), 2));
             sp.E1 = R_s;
             sp.E2 = cx(-R_p.re, -R_p.im);
@@ -575,7 +581,7 @@ RPX_DEV void eval_children(const rpx_material_t &m, const Ray &in, uint32_t idx,
             emit(sp);
         }
         const Cx T_s = cmul(k.ts, E1), T_p = cmul(k.tp, E2);
-        if (n3.re * (cnorm2(T_s) + cnorm2(T_p)) * per_P > m.transmission_threshold) {
+        if (passes(n3.re * (cnorm2(T_s) + cnorm2(T_p)), P_in, m.transmission_threshold)) {
             sp.direction = sub(tg2, mul(normal, inward ? c2 : -c2));
             sp.E1 = T_s;
             sp.E2 = T_p;

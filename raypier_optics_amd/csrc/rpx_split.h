@@ -401,7 +401,6 @@ RPX_DEV void eval_children_split(const rpx_material_t &m, const RayS &in, double
         const Cf n1 = cf_of(n1d), n3 = cf_of(n3d);
         const float P_in = n1.re * (cfabs2(E1) + cfabs2(E2));
         if (P_in == 0.0f) return;
-        const float per_P = 1.0f / P_in;
         const V3 tangent = sub(in_dir, mul(normal, cosTheta));
         const V3 tg2 = mul(tangent, n1d.re / n3d.re);
         const double tan_mag_sq = mag_sq(tg2);
@@ -427,7 +426,7 @@ RPX_DEV void eval_children_split(const rpx_material_t &m, const RayS &in, double
                 return;
         }
         const Cf R_s = cfmul(k.rs, E1), R_p = cfmul(k.rp, E2);
-        if (n1.re * (cfabs2(R_s) + cfabs2(R_p)) * per_P > (float)m.reflection_threshold) {
+        if (passes(n1.re * (cfabs2(R_s) + cfabs2(R_p)), P_in, (float)m.reflection_threshold)) {
             sp.direction = f3_of(reflect_dir(in_dir, normal, cosTheta));
             sp.E1 = R_s;
             sp.E2 = cfneg(R_p);
@@ -436,7 +435,7 @@ RPX_DEV void eval_children_split(const rpx_material_t &m, const RayS &in, double
             emit(sp);
         }
         const Cf T_s = cfmul(k.ts, E1), T_p = cfmul(k.tp, E2);
-        if (n3.re * (cfabs2(T_s) + cfabs2(T_p)) * per_P > (float)m.transmission_threshold) {
+        if (passes(n3.re * (cfabs2(T_s) + cfabs2(T_p)), P_in, (float)m.transmission_threshold)) {
             sp.direction = f3_of(sub(tg2, mul(normal, inward ? c2 : -c2)));
             sp.E1 = T_s;
             sp.E2 = T_p;
