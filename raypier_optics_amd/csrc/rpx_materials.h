@@ -305,16 +305,18 @@ RPX_DEV Coefs fresnel_coefs(Cx n1, Cx n2, double cos1, double sin1, bool real, d
 // and a^2 - b^2 is a product again: 4 n1 cos1 n2 cos2 e^-phi over the same
 // denominator for s, 4 n1 cos2 n2 cos1 e^-phi for p.  Three real indices below
 // total reflection (`real`): e^phi has modulus 1 and the rest is real.
+// `n2c2sq`, (n2 cos2)^2 = n2^2 - n1^2 sin1^2, is then above zero as computed, so
+// that no rounding of sin2^2 takes cos2 to zero or past it.
 RPX_DEV Coefs film_coefs(Cx n1, Cx n2, Cx n3, double cos1, double sin1, double dwc, bool real, double sin1sq,
-                         double cos3r) {
+                         double n2c2sq, double cos3r) {
     Coefs o;
     if (real) {
-        const double q = n1.re / n2.re, sin2sq = sin1sq * q * q;
-        const double cos2 = sqrt(1.0 - sin2sq);
+        const double inv2 = 1.0 / n2.re, q = n1.re * inv2, sin2sq = sin1sq * q * q;
+        const double n2c2 = sqrt(n2c2sq), cos2 = n2c2 * inv2;
         double sp, cp;   // e^-phi = cp + i sp
         sincos(dwc * (n2.re - sin2sq) / cos2, &sp, &cp);
         const double er = fma(cp, cp, -(sp * sp)), ei = 2.0 * sp * cp;   // e^-2phi
-        const double n1c1 = n1.re * cos1, n2c2 = n2.re * cos2, n3c3 = n3.re * cos3r;
+        const double n1c1 = n1.re * cos1, n3c3 = n3.re * cos3r;
         const double n1c2 = n1.re * cos2, n2c1 = n2.re * cos1, n2c3 = n2.re * cos3r, n3c2 = n3.re * cos2;
         const double aspect = 4.0 * sqrt(cos3r / cos1);
         auto pol = [&](double a, double b, double c, double d, double t, Cx &r_out, Cx &t_out) {
@@ -558,10 +560,10 @@ RPX_DEV void eval_children(const rpx_material_t &m, const Ray &in, uint32_t idx,
         if (film) {
             if constexpr ((F & M_COATED) != 0) {
                 const double sin1sq = mag_sq(tangent);
-                real = real && sd.n_coat.im == 0.0 && sd.n_coat.re > 0.0 &&
-                       n1.re * n1.re * sin1sq < sd.n_coat.re * sd.n_coat.re;
+                const double n2c2sq = sd.n_coat.re * sd.n_coat.re - n1.re * n1.re * sin1sq;
+                real = real && sd.n_coat.im == 0.0 && sd.n_coat.re > 0.0 && n2c2sq > 0.0;
                 k = film_coefs(n1, sd.n_coat, n3, cos1, sqrt(fabs(1 - cos1 * cos1)),
-                               2 * M_PI * m.thickness / wavelength, real, sin1sq, c2);
+                               2 * M_PI * m.thickness / wavelength, real, sin1sq, n2c2sq, c2);
             } else {
                 return;
             }

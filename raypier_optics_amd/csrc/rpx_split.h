@@ -193,16 +193,18 @@ RPX_DEV CoefsS fresnel_coefs_s(Cf n1, Cf n2, float cos1, float sin1, bool real, 
     return c;
 }
 
+// As film_coefs; n2c2sq comes from float64, where the last digits of an angle
+// near the film's critical one are.
 RPX_DEV CoefsS film_coefs_s(Cf n1, Cf n2, Cf n3, float cos1, float sin1, float dwc, bool real, float sin1sq,
-                            float cos3r) {
+                            float n2c2sq, float cos3r) {
     CoefsS o;
     if (real) {
-        const float q = n1.re / n2.re, sin2sq = sin1sq * q * q;
-        const float cos2 = sqrtf(1.0f - sin2sq);
+        const float inv2 = 1.0f / n2.re, q = n1.re * inv2, sin2sq = sin1sq * q * q;
+        const float n2c2 = sqrtf(n2c2sq), cos2 = n2c2 * inv2;
         float sp, cp;
         sincosf(dwc * (n2.re - sin2sq) / cos2, &sp, &cp);
         const float er = cp * cp - sp * sp, ei = 2.0f * sp * cp;
-        const float n1c1 = n1.re * cos1, n2c2 = n2.re * cos2, n3c3 = n3.re * cos3r;
+        const float n1c1 = n1.re * cos1, n3c3 = n3.re * cos3r;
         const float n1c2 = n1.re * cos2, n2c1 = n2.re * cos1, n2c3 = n2.re * cos3r, n3c2 = n3.re * cos2;
         const float aspect = 4.0f * sqrtf(cos3r / cos1);
         auto pol = [&](float a, float b, float c, float d, float t, Cf &r_out, Cf &t_out) {
@@ -412,10 +414,10 @@ RPX_DEV void eval_children_split(const rpx_material_t &m, const RayS &in, double
             if constexpr ((F & M_COATED) != 0) {
                 const Cf n2 = cf_of(sd.n_coat);
                 const double sin1sq = mag_sq(tangent);
-                real = real && n2.im == 0.0f && n2.re > 0.0f &&
-                       n1d.re * n1d.re * sin1sq < sd.n_coat.re * sd.n_coat.re;
+                const double n2c2sq = sd.n_coat.re * sd.n_coat.re - n1d.re * n1d.re * sin1sq;
+                real = real && n2.im == 0.0f && n2.re > 0.0f && n2c2sq > 0.0;
                 k = film_coefs_s(n1, n2, n3, cos1, sin1, (float)(2 * M_PI * m.thickness / wavelength), real,
-                                 (float)sin1sq, (float)c2);
+                                 (float)sin1sq, (float)n2c2sq, (float)c2);
             } else {
                 return;
             }
