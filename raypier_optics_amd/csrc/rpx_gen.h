@@ -18,6 +18,9 @@ namespace rpx {
 #define RPX_LDS_FACES 64
 #define RPX_LDS_LISTS 16
 #define RPX_BLOCK 256
+// Lens chains and served steps of at least this many rays take 512-ray tiles
+// (gen_block in rpx_trace.hip says why there).
+#define RPX_LARGE_TILE_RAYS 69632
 
 // ------------------------------------------------------------ workspace
 // Generation control words (device), cleared by k_clear before each

@@ -74,9 +74,14 @@ struct BatchControl {
 };
 
 // Rays per tile of a step: as the chains' (gen_block in rpx_trace.hip), 512 for
-// the lens variants in steps of at least 65,536 rays (24 lens jobs of up to
-// 500,000 rays: 282 -> 235 us per tile kernel), else 256.  Moment partials are
-// kept per 256 rays either way, so that a job's sums do not depend on the size.
+// the lens variants in steps of at least RPX_LARGE_TILE_RAYS rays (24 lens jobs of
+// up to 500,000 rays: 282 -> 235 us per tile kernel), else 256.  The rays are the
+// sum over the step's jobs, each of which fills up its own last tile, so many
+// small jobs gain less: tile kernels of a whole run, 256- against 512-ray tiles,
+// 64 jobs of 1,100 rays 800 / 809 us, 24 of 3,000 774 / 788, 8 of 9,000 766 / 753,
+// 4 of 20,000 834 / 776, 2 of 45,000 915 / 840, 64 of 1,600 888 / 843, 64 of 5,000
+// 1,444 / 1,298.  Moment partials are kept per 256 rays either way, so that a
+// job's sums do not depend on the size.
 #define BATCH_SMALL 256
 #define BATCH_LARGE 512
 
@@ -726,7 +731,7 @@ extern "C" rpx_status_t rpx_server_step(rpx_server_t *s, rpx_job_result_t *finis
             b.counts = s->d_counts + j->slot * RPX_SERVE_COUNT_WORDS;
             if (j->variant == V_ALL || (j->variant == V_LENS && variant == V_SPHERES)) variant = j->variant;
         }
-        const uint64_t B = variant != V_ALL && rays >= 65536 ? BATCH_LARGE : BATCH_SMALL;
+        const uint64_t B = variant != V_ALL && rays >= RPX_LARGE_TILE_RAYS ? BATCH_LARGE : BATCH_SMALL;
         tile = 0;
         for (size_t k = 0; k < batch.size(); ++k) {
             s->h_jobs[k].tile_begin = tile;

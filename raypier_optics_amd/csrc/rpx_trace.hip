@@ -861,13 +861,19 @@ void k_generation(TraceArgs A) {
 // Rays per tile of a float64 chain.  Two 512-lane workgroups fill a CU at the
 // lens variants' four waves per SIMD, and their tiles halve the look-backs and
 // the staging: 4,194,304 rays of the asphere and doublet 0.54 -> 0.48 ms per
-// generation (1,024-ray tiles: 0.49 ms); a lens of six surfaces, kernels per
-// trace, 256- against 512-ray tiles: 8,000 rays 114 / 124 us, 65,536 rays 156 /
-// 160, 100,000 rays 172 / 160, 200,000 rays 225 / 211.  V_ALL keeps 256: its three
-// waves per SIMD leave a 512-lane workgroup's second one no room (Michelson:
-// 25 % slower).
+// generation (1,024-ray tiles: 0.49 ms).  Up to 65,536 rays there is a 256-ray tile
+// for every CU and all of them end together; a few more, and some CUs get a second
+// one.  Kernels per trace, 256- against 512-ray tiles, us:
+//   rays     8,000    32,768   65,536   68,000   70,000   73,728   98,304   200,003
+//   lens 1   99/110  131/131  141/146  136/136  137/135  155/150  172/156  214/200
+//   lens 2  127/139  153/157  164/173  175/174  178/175  186/177  205/187  291/266
+//   doublet  79/87    95/97   102/108  111/111  113/113  119/113  127/116  182/166
+//   singlet  57/64    74/75    96/95   100/91    99/93   102/98   119/113  195/177
+// (two aspheric lenses of six surfaces, the asphere and doublet, the biconvex
+// singlet.)  V_ALL keeps 256: its three waves per SIMD leave a 512-lane workgroup's
+// second one no room (Michelson: 25 % slower).
 static uint32_t gen_block(uint32_t variant, uint64_t n_in) {
-    return variant != V_ALL && n_in >= 65536 ? 512u : 256u;
+    return variant != V_ALL && n_in >= RPX_LARGE_TILE_RAYS ? 512u : 256u;
 }
 
 template <int B>

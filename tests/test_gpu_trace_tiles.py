@@ -1,4 +1,4 @@
-"""Traces either side of the tile-size rule (512-ray tiles from 65,536 input
+"""Traces either side of the tile-size rule (512-ray tiles from 69,632 input
 rays on, 256 below): one call equals the concatenation of calls on pieces of
 the input, all of which take the small tiles, to the last bit.  Both run the
 same code per ray, and children keep their parents' order, so nothing but the
@@ -21,7 +21,7 @@ def _trace(rays, w, depth):
 
 
 @pytest.mark.parametrize("system", ["spheres", "aspheres"])
-@pytest.mark.parametrize("n", [65535, 65536, 65537, 66049, 98303])
+@pytest.mark.parametrize("n", [65535, 65536, 65537, 66049, 69631, 69632, 69633, 70145, 98303])
 def test_tile_sizes_agree(gpu, system, n):
     if system == "spheres":
         w, depth = workloads.singlet_c1(n), 4
