@@ -1,8 +1,11 @@
 // Face intersection, normals, aperture shapes and Zernike distortions (FP64).
 //
-// Each routine follows the arithmetic of the reference face it stands in for;
-// the reference line is cited beside it.  `is_base` is the reference's
-// is_base_ray flag: parabasal rays skip most aperture tests.
+// Each routine solves the equation of the reference face it stands in for, whose
+// line is cited beside it, and takes its decisions (root choice, range and
+// aperture tests, when a root search gives up) as it does; the arithmetic is its
+// own, equal to a few ulp.  rpx_faces_ref.h has the intersections with the
+// reference's roundings.  `is_base` is the reference's is_base_ray flag:
+// parabasal rays skip most aperture tests.
 #pragma once
 #include "rpx_internal.h"
 

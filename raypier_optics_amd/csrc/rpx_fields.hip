@@ -5,10 +5,11 @@
 //                 the closed-form 3x3 least-squares mode fit
 //                 (evaluate_one_mode, cfields.pyx:156-215).
 //   k_field_prep  per-gausslet invariants of sum_gaussian_modes
-//                 (cfields.pyx:76-99) into a structure-of-arrays table.
-//   k_field_sum   one evaluation point per lane; gausslet invariants stream
-//                 through LDS in tiles and every lane sums them in gausslet
-//                 order, so each point's sum has the reference's order.
+//                 (cfields.pyx:76-99), one 288-byte record per gausslet.
+//   k_field_sum   one evaluation point per lane; the gausslet is the same in
+//                 every lane, so its record comes by scalar loads into SGPRs.
+//                 A lane sums a chunk of gausslets in order; k_field_reduce
+//                 adds the chunks' sums in a fixed order.
 #include <hip/hip_runtime.h>
 #include <mutex>
 #include <algorithm>

@@ -147,10 +147,11 @@ static __device__ __forceinline__ uint32_t block_scan_small(uint32_t c, uint32_t
 
 // --------------------------------------------------- single-pass generation
 // One launch per ray generation: intersect, evaluate the material once, and
-// place the children with a decoupled look-back scan over tiles of RPX_BLOCK
-// rays.  Tiles are handed out by an atomic counter in launch order, so every
-// tile a workgroup waits for belongs to a workgroup that is already running;
-// the wait is also bounded by a poll limit (error flag instead of a hang).
+// place the children with a decoupled look-back scan over tiles of rays.  With
+// tiles handed out by an atomic counter every tile a workgroup waits for belongs
+// to a workgroup that is already running; with tiles in launch order (chains) the
+// wait is bounded in time (run_chain).  Either wait is also bounded by a poll
+// limit (error flag instead of a hang).
 
 #define RPX_LOOKBACK_POLLS (1u << 22)
 // A status word: flag (bits 62-63) | tag (bits 48-61) | value (bits 0-47).

@@ -1,10 +1,12 @@
 // Device-side types and arithmetic helpers for the gfx950 tracer.
 //
-// All FP64 routines keep the operation order of the reference Cython code
-// (raypier/core/ctracer.pyx:83-262 vector maths, cmaterials.pyx complex maths)
-// and the library is compiled with -ffp-contract=off, so that add/mul/div/sqrt
-// chains round exactly like the reference's x86-64 build.  Only libm-level
-// functions (pow, sin, cos, atan2, exp, hypot) may differ by an ulp.
+// The float64 sources are compiled with -ffp-contract=off: a product and a sum
+// are fused only where the code says fma.  The vector and complex helpers that
+// cite the reference (raypier/core/ctracer.pyx:83-262, cmaterials.pyx) keep its
+// operation order and round as its x86-64 build does; the face tests of
+// rpx_faces_ref.h rest on them.  The traces' own code (rpx_faces.h,
+// rpx_materials.h) and the helpers below without a citation reach the same
+// values to a few ulp in fewer operations.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -85,7 +87,6 @@ struct Cx {
 RPX_DEV Cx cx(double r, double i) { Cx c; c.re = r; c.im = i; return c; }
 RPX_DEV Cx cadd(Cx a, Cx b) { return cx(a.re + b.re, a.im + b.im); }
 RPX_DEV Cx csub(Cx a, Cx b) { return cx(a.re - b.re, a.im - b.im); }
-RPX_DEV Cx cneg(Cx a) { return cx(-a.re, -a.im); }
 RPX_DEV Cx cmul(Cx a, Cx b) {
     return cx(a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re);
 }
@@ -107,7 +108,6 @@ RPX_DEV Cx cdiv(Cx n, Cx d) {
     }
     return cx(x, y);
 }
-RPX_DEV double cabs_(Cx a) { return hypot(a.re, a.im); }
 // Principal square root (Kahan's formulation).
 RPX_DEV Cx csqrt_(Cx z) {
     double x = z.re, y = z.im;

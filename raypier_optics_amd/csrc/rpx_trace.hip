@@ -1,13 +1,15 @@
 // Generation tracer for gfx950: one generation of rays (or gausslets) against
 // a device-resident scene, with stable parent-major compaction of children.
 //
-// One launch per generation (after k_clear): each workgroup takes a tile of
-// 256 rays, runs the nearest-face search (scene staged in LDS), updates the
-// parents in place (length, end_face_idx), counts face hits, evaluates the
-// material, and places the children by a decoupled look-back over the tiles
-// in parent-major order (k_generation for rays; k_gausslet_generation for
-// gausslets, which builds children and parabasal rays after the look-back).
-// rpx_trace_rays chains the ray generations on the device (rpx_gen.h).
+// One launch per generation: each workgroup takes a tile of 256 or 512 rays
+// (gen_block; gausslets 256), runs the nearest-face search (scene staged in LDS),
+// updates the parents in place (length, end_face_idx), counts face hits, evaluates
+// the material once, keeping up to two children in registers, and places them by
+// a decoupled look-back over the tiles in parent-major order (k_generation for
+// rays; k_gausslet_generation for gausslets, whose children's parabasal rays are
+// built after the look-back).  rpx_trace_rays and rpx_trace_gausslets chain the
+// generations on the device (rpx_gen.h); the one-generation entry points clear
+// the tile status first (k_clear).
 #include <hip/hip_runtime.h>
 #include <atomic>
 #include <algorithm>
